@@ -10,18 +10,16 @@
 // |i'-i| <= hx, |j'-j| <= hy(j), with w = exp(-delta^2/(2 sigma^2)) and
 // delta the haversine distance in degrees.  On the reference's grids (uniform
 // axes from arange) a weight depends on the row pair (j, j') and the column
-// offset |i'-i| only, up to the rounding of lon(i')-lon(i): one workgroup
-// owns an output row, evaluates the (hx+1) weights of each window row j'
-// once into LDS, stages data row j' in LDS, and every thread accumulates its
-// cells in the reference's order (j' outer, i' inner, ascending).  The
-// transcendental work is thus per (j, j', offset), not per (cell, node); the
-// per-node work is one LDS read, one multiply and two adds in FP64.  The
-// latitude terms sin((lat-lat')/2)^2, cos(lat), cos(lat') are the
-// reference's per pair; the longitude term is sin(dlon_k/2)^2 with dlon_k =
-// lon(k)-lon(0).
+// offset |i'-i| only, up to the rounding of lon(i')-lon(i): the weights of a
+// row pair are evaluated once per column offset, not per (cell, node), and
+// the per-node work is one fused multiply-add in FP64 on register operands
+// (k_smooth_geo2).  The latitude term sin((lat-lat')/2)^2 is the reference's
+// per pair; the longitude term is sin(dlon_k/2)^2 with dlon_k = lon(k)-lon(0).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
+#include <type_traits>
 
 #include "satt_internal.h"
 
@@ -42,220 +40,352 @@ __global__ void k_geo_s2(const double *lon, int nx, double *s2) {
   s2[k] = s * s;
 }
 
-// One workgroup per (output row j, field f).  LDS: the row pair's weights
-// w[0..hxe] and data row j' (nx each).  CPT cells per thread: i = tid + q*bs,
-// MAXT threads at most (512 when a thread has several cells, which leaves it
-// the registers of its accumulators).
-template <int CPT, int MAXT>
-__global__ __launch_bounds__(MAXT) void k_smooth_geo2(GeoSmooth P) {
-  extern __shared__ double lds[];
-  const int j = blockIdx.x, f = blockIdx.y;
-  const int nx = P.nx, ny = P.ny, bs = blockDim.x, tid = threadIdx.x;
-  const int hx = P.hx[f], hy = P.hy[(size_t)f * ny + j];
-  const int hxe = hx < nx - 1 ? hx : nx - 1;
-  double *wl = lds, *dl = lds + nx;
-  const double *data = P.data + (P.ndata == 1 ? 0 : (size_t)f * nx * ny);
-  const double sig = P.sigma[f], two_sig_sq = 2.0 * (sig * sig);
-  const int n1 = j - hy > 0 ? j - hy : 0, n2 = j + hy < ny - 1 ? j + hy : ny - 1;
-  const double c0 = cos(P.lat[j] * kGeoDeg2Rad);
-  double swd[CPT], sw[CPT];
-#pragma unroll
-  for (int q = 0; q < CPT; ++q) swd[q] = sw[q] = 0.0;
-  for (int jj = n1; jj <= n2; ++jj) {
-    const double c1 = cos(P.lat[jj] * kGeoDeg2Rad);
-    const double sl = sin((P.lat[j] - P.lat[jj]) * kGeoDeg2Rad * 0.5);
-    const double sdl = sl * sl;
-    for (int k = tid; k <= hxe; k += bs) {
-      const double a = sdl + P.s2[k] * c0 * c1;
-      const double deg = 2.0 * atan2(sqrt(a), sqrt(1.0 - a));
-      const double delta = kGeoRadius * deg * kGeoKm2Deg;
-      wl[k] = exp(-(delta * delta) / two_sig_sq);
-    }
-    const double *row = data + (size_t)jj * nx;
-    for (int i = tid; i < nx; i += bs) dl[i] = row[i];
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < CPT; ++q) {
-      const int i = tid + q * bs;
-      if (i < nx) {
-        const int k0 = -hx > -i ? -hx : -i, k1 = hx < nx - 1 - i ? hx : nx - 1 - i;
-        const double *dp = dl + i;
-        double a = swd[q], b = sw[q];
-        // offsets in ascending order, split at 0 so that both the weight and
-        // the data index run linearly; eight nodes' loads are issued before
-        // their sums, so one LDS round trip serves eight nodes
-        int k = k0;
-        for (; k + 8 <= 0; k += 8) {
-          double w[8], d[8];
-#pragma unroll
-          for (int u = 0; u < 8; ++u) {
-            w[u] = wl[-(k + u)];
-            d[u] = dp[k + u];
-          }
-#pragma unroll
-          for (int u = 0; u < 8; ++u) {
-            a += w[u] * d[u];
-            b += w[u];
-          }
-        }
-        for (; k < 0; ++k) {
-          const double w = wl[-k];
-          a += w * dp[k];
-          b += w;
-        }
-        for (; k + 8 <= k1 + 1; k += 8) {
-          double w[8], d[8];
-#pragma unroll
-          for (int u = 0; u < 8; ++u) {
-            w[u] = wl[k + u];
-            d[u] = dp[k + u];
-          }
-#pragma unroll
-          for (int u = 0; u < 8; ++u) {
-            a += w[u] * d[u];
-            b += w[u];
-          }
-        }
-        for (; k <= k1; ++k) {
-          const double w = wl[k];
-          a += w * dp[k];
-          b += w;
-        }
-        swd[q] = a;
-        sw[q] = b;
-      }
-    }
-    __syncthreads();
-  }
-  double *out = P.out + (size_t)f * nx * ny + (size_t)j * nx;
-#pragma unroll
-  for (int q = 0; q < CPT; ++q) {
-    const int i = tid + q * bs;
-    if (i < nx) out[i] = (0.0 + swd[q]) / sw[q];
+// The lat-lon haversine a = sin^2(theta/2) of a window node as the exponent
+// of its weight, theta^2 * kap / 4 with kap = 4 (R km2deg)^2 / (2 sigma^2).
+// SMALL: theta^2 = 4 asin(sqrt(a))^2 by its power series, 4a (1 + a/3 +
+// 8a^2/45 + ...), eight terms: for a <= kSmallA the next one is below 1e-18
+// of the sum.  It takes 9 operations where the atan2 and the two square
+// roots of the general form take about 150, which had been a quarter of the
+// kernel's arithmetic at wide windows.
+constexpr double kSmallA = 1.0 / 128;
+template <bool SMALL>
+__device__ __forceinline__ double geo_weight(double a, double kap) {
+  if constexpr (SMALL) {
+    double p = 512.0 / 12870;
+    p = __builtin_fma(p, a, 1024.0 / 21021);
+    p = __builtin_fma(p, a, 128.0 / 2079);
+    p = __builtin_fma(p, a, 128.0 / 1575);
+    p = __builtin_fma(p, a, 4.0 / 35);
+    p = __builtin_fma(p, a, 8.0 / 45);
+    p = __builtin_fma(p, a, 1.0 / 3);
+    p = __builtin_fma(p, a, 1.0);
+    return exp(-(kap * (a * p)));
+  } else {
+    const double t = atan2(sqrt(a), sqrt(1.0 - a));
+    return exp(-(kap * (t * t)));
   }
 }
 
-// Two output rows (j, j+1) per workgroup, one cell per thread (nx <= 1024):
-// each staged data row serves both rows, so a node costs three LDS reads for
-// two cells (the two rows' weights and the shared datum) instead of four, and
-// a window row takes one barrier for two output rows.  Each cell's sums keep
-// the single-row kernel's order (window rows ascending, offsets ascending).
-__global__ __launch_bounds__(1024) void k_smooth_geo2_pair(GeoSmooth P) {
-  extern __shared__ double lds[];
-  const int j0 = 2 * blockIdx.x, f = blockIdx.y;
-  const int nx = P.nx, ny = P.ny, tid = threadIdx.x;
-  const bool two = j0 + 1 < ny;
-  const int hx = P.hx[f];
-  const int hy0 = P.hy[(size_t)f * ny + j0], hy1 = two ? P.hy[(size_t)f * ny + j0 + 1] : 0;
-  const int hxe = hx < nx - 1 ? hx : nx - 1;
-  double *w0 = lds, *w1 = lds + nx, *dl = lds + 2 * nx;
-  const double *data = P.data + (P.ndata == 1 ? 0 : (size_t)f * nx * ny);
-  const double sig = P.sigma[f], two_sig_sq = 2.0 * (sig * sig);
-  const int a1 = j0 - hy0 > 0 ? j0 - hy0 : 0, a2 = j0 + hy0 < ny - 1 ? j0 + hy0 : ny - 1;
-  const int b1 = two ? (j0 + 1 - hy1 > 0 ? j0 + 1 - hy1 : 0) : a1;
-  const int b2 = two ? (j0 + 1 + hy1 < ny - 1 ? j0 + 1 + hy1 : ny - 1) : a2;
-  const int n1 = a1 < b1 ? a1 : b1, n2 = a2 > b2 ? a2 : b2;
-  const double c00 = cos(P.lat[j0] * kGeoDeg2Rad);
-  const double c01 = two ? cos(P.lat[j0 + 1] * kGeoDeg2Rad) : c00;
-  const int i = tid;
-  const int k0 = -hx > -i ? -hx : -i, k1 = hx < nx - 1 - i ? hx : nx - 1 - i;
-  double s0 = 0.0, t0 = 0.0, s1 = 0.0, t1 = 0.0;
-  for (int jj = n1; jj <= n2; ++jj) {
-    const bool in0 = jj >= a1 && jj <= a2, in1 = two && jj >= b1 && jj <= b2;
-    const double c1 = cos(P.lat[jj] * kGeoDeg2Rad);
-    // the weights of both rows: lanes 0..hxe for row j0, the next hxe+1 for j0+1
-    for (int q = tid; q <= 2 * hxe + 1; q += blockDim.x) {
-      const int r = q > hxe, k = r ? q - hxe - 1 : q;
-      if (r ? !in1 : !in0) continue;
-      const double latj = P.lat[j0 + r], cj = r ? c01 : c00;
-      const double sl = sin((latj - P.lat[jj]) * kGeoDeg2Rad * 0.5);
-      const double a = sl * sl + P.s2[k] * cj * c1;
-      const double deg = 2.0 * atan2(sqrt(a), sqrt(1.0 - a));
-      const double delta = kGeoRadius * deg * kGeoKm2Deg;
-      (r ? w1 : w0)[k] = exp(-(delta * delta) / two_sig_sq);
+// num[r][c] += sum over k = 0 .. n - 1, ascending, of w[k*RW + r] *
+// d(c + DIR*k), for a lane's C consecutive cells c and RR output rows; d is
+// the staged data row at the lane's first cell.  The cells' data slide
+// through a ring of C+3 registers: per offset a lane reads one datum and RR
+// weights from LDS for RR*C products.  Reads run up to C+2 elements past the
+// last one used (kPadC below).
+template <int RR, int RW, int C, int DIR>
+__device__ __forceinline__ void smooth_side(const double *w, const double *d, int n,
+                                            double (&num)[RR][C]) {
+  constexpr int K = C + 3;
+  const double *p = DIR > 0 ? d : d + (C - 1);
+  double a[RR][C] = {}, v[K], wq[2][RR];  // wq: this offset's weights, the next one's
+#pragma unroll
+  for (int x = 0; x < K; ++x) v[x] = p[DIR * x];
+#pragma unroll
+  for (int r = 0; r < RR; ++r) wq[0][r] = w[r];
+  static_assert(K % 2 == 0, "wq alternates");
+  auto at = [&](int u, int k) {
+    const double vn = p[DIR * (k + u + K)];
+#pragma unroll
+    for (int r = 0; r < RR; ++r) wq[(u + 1) & 1][r] = w[(k + u + 1) * RW + r];
+#pragma unroll
+    for (int r = 0; r < RR; ++r)
+#pragma unroll
+      for (int e = 0; e < C; ++e) {
+        const int c = DIR > 0 ? e : C - 1 - e;
+        a[r][c] = __builtin_fma(wq[u & 1][r], v[(u + e) % K], a[r][c]);
+      }
+    v[u] = vn;
+  };
+  int k = 0;
+  for (; k + K <= n; k += K) {
+#pragma unroll
+    for (int u = 0; u < K; ++u) at(u, k);
+  }
+  const int rem = n - k;
+#pragma unroll
+  for (int u = 0; u < K - 1; ++u)
+    if (u < rem) at(u, k);
+#pragma unroll
+  for (int r = 0; r < RR; ++r)
+#pragma unroll
+    for (int c = 0; c < C; ++c) num[r][c] = num[r][c] + a[r][c];
+}
+
+// Orders a wave's LDS accesses for the compiler (the hardware runs one wave's
+// LDS instructions in order, and every wave here uses its own part of it).
+__device__ __forceinline__ void lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// The smoothing is sum(w*data)/sum(w): k_smooth_norm forms the denominators
+// of each distinct sigma, k_smooth_geo2 the numerators and the quotients.
+// Both take the window rows j' in S waves (wave j' mod S, added in wave
+// order) and a row's offsets in ascending distance, one side after the other:
+//   num += sum_{k>=1} w[k] d(i+k), then + sum_{k>=1} w[k] d(i-k), then + w[0] d(i)
+//   den += P[min(hx, nx-1-i)],     then + P[min(hx, i)],          then + w[0]
+// with P[m] the running sums of w[1..m]: on a field of ones the numerator takes the
+// denominator's own operations, so that constants are kept exactly.
+constexpr int kMaxSplit = 4;
+
+// The latitude terms of a wave's window rows, 64 of them at a time, one per
+// lane: cos(lat') and, for each output row, sin((lat - lat')/2)^2.
+template <int RW>
+struct LatTerms {
+  double c1 = 0, sdl[RW] = {};
+  int left = 0;
+  // the terms of row jj (the wave's rows are S apart): cos(lat)cos(lat') and
+  // the squared sine of every output row
+  __device__ __forceinline__ void at(const GeoSmooth &P, int jj, int S, int lane,
+                                     const double (&lat)[RW], const double (&cl)[RW],
+                                     double (&cc)[RW], double (&sd)[RW]) {
+    if (left == 0) {
+      const int jl = jj + S * lane;
+      const double latj = P.lat[jl < P.ny ? jl : P.ny - 1];
+      c1 = cos(latj * kGeoDeg2Rad);
+#pragma unroll
+      for (int r = 0; r < RW; ++r) {
+        const double sl = sin((lat[r] - latj) * kGeoDeg2Rad * 0.5);
+        sdl[r] = sl * sl;
+      }
+      left = 64;
     }
-    const double *row = data + (size_t)jj * nx;
-    for (int q = tid; q < nx; q += blockDim.x) dl[q] = row[q];
-    __syncthreads();
-    if (i < nx) {
-      const double *dp = dl + i;
-      if (in0 && in1) {
-        // four nodes' loads (twelve LDS reads) are issued before their sums
-        int k = k0;
-        for (; k + 4 <= 0; k += 4) {
-          double d[4], x0[4], x1[4];
+    const int src = 64 - left--;
+    const double cj = __shfl(c1, src, 64);
 #pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            d[u] = dp[k + u];
-            x0[u] = w0[-(k + u)];
-            x1[u] = w1[-(k + u)];
-          }
+    for (int r = 0; r < RW; ++r) {
+      sd[r] = __shfl(sdl[r], src, 64);
+      cc[r] = cl[r] * cj;
+    }
+  }
+};
+
+__device__ __forceinline__ double geo_kap(double sig) {
+  return 4.0 * (kGeoRadius * kGeoKm2Deg) * (kGeoRadius * kGeoKm2Deg) / (2.0 * (sig * sig));
+}
+// the wave sw's first window row at or after n1
+__device__ __forceinline__ int first_row(int n1, int sw, int S) {
+  return n1 + ((sw - n1) % S + S) % S;
+}
+
+// Denominators of RN output rows, a tile of 64*kNormC columns, one sigma per
+// workgroup of S waves.  A wave evaluates its window rows' weights, one lane
+// per output row turns them into running sums, and every lane adds the two
+// its columns need.
+constexpr int kNormC = 7;
+template <int RN, bool SMALL>
+__global__ __launch_bounds__(64 * kMaxSplit) void k_smooth_norm(GeoSmooth P, int lds_wave) {
+  extern __shared__ double lds[];
+  const int lane = threadIdx.x & 63;
+  const int S = blockDim.x >> 6, sw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int j0 = RN * blockIdx.x, f = P.norm_field[blockIdx.y], i0 = 64 * kNormC * blockIdx.z;
+  const int nx = P.nx, ny = P.ny;
+  const int hx = P.hx[f], hxe = hx < nx - 1 ? hx : nx - 1;
+  const int ld = (hxe + 1) | 1;  // odd: the running-sum lanes read different banks
+  double *wl = lds + (size_t)sw * lds_wave;
+  const double kap = geo_kap(P.sigma[f]);
+  int lo[RN], hi[RN], n1 = ny, n2 = -1;
+  double latr[RN], cr[RN];
 #pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            s0 += x0[u] * d[u];
-            t0 += x0[u];
-            s1 += x1[u] * d[u];
-            t1 += x1[u];
-          }
-        }
-        for (; k < 0; ++k) {
-          const double d = dp[k], x0 = w0[-k], x1 = w1[-k];
-          s0 += x0 * d;
-          t0 += x0;
-          s1 += x1 * d;
-          t1 += x1;
-        }
-        for (; k + 4 <= k1 + 1; k += 4) {
-          double d[4], x0[4], x1[4];
+  for (int r = 0; r < RN; ++r) {
+    const int j = j0 + r < ny ? j0 + r : ny - 1, hy = P.hy[(size_t)f * ny + j];
+    lo[r] = j - hy > 0 ? j - hy : 0;
+    hi[r] = j + hy < ny - 1 ? j + hy : ny - 1;
+    n1 = lo[r] < n1 ? lo[r] : n1;
+    n2 = hi[r] > n2 ? hi[r] : n2;
+    latr[r] = P.lat[j];
+    cr[r] = cos(latr[r] * kGeoDeg2Rad);
+  }
+  double den[RN][kNormC] = {};
+  LatTerms<RN> T;
+  for (int jj = first_row(n1, sw, S); jj <= n2; jj += S) {
+    double cc[RN], sd[RN], w0[RN];
+    T.at(P, jj, S, lane, latr, cr, cc, sd);
+    lds_order();  // the previous row's sums have been read
+    for (int k = lane; k <= hxe; k += 64) {
+      const double s2 = P.s2[k];
 #pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            d[u] = dp[k + u];
-            x0[u] = w0[k + u];
-            x1[u] = w1[k + u];
-          }
+      for (int r = 0; r < RN; ++r)
+        wl[r * ld + k] = geo_weight<SMALL>(__builtin_fma(s2, cc[r], sd[r]), kap);
+    }
+    lds_order();
 #pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            s0 += x0[u] * d[u];
-            t0 += x0[u];
-            s1 += x1[u] * d[u];
-            t1 += x1[u];
-          }
-        }
-        for (; k <= k1; ++k) {
-          const double d = dp[k], x0 = w0[k], x1 = w1[k];
-          s0 += x0 * d;
-          t0 += x0;
-          s1 += x1 * d;
-          t1 += x1;
-        }
-      } else {
-        const double *w = in0 ? w0 : w1;
-        double s = in0 ? s0 : s1, t = in0 ? t0 : t1;
-        int k = k0;
-        for (; k < 0; ++k) {
-          const double x = w[-k];
-          s += x * dp[k];
-          t += x;
-        }
-        for (; k <= k1; ++k) {
-          const double x = w[k];
-          s += x * dp[k];
-          t += x;
-        }
-        if (in0) {
-          s0 = s;
-          t0 = t;
-        } else {
-          s1 = s;
-          t1 = t;
+    for (int r = 0; r < RN; ++r) w0[r] = wl[r * ld];
+    if (lane < RN) {
+      double *w = wl + lane * ld, s = 0.0;
+      w[0] = 0.0;
+      int k = 1;
+      for (; k + 8 <= hxe + 1; k += 8) {
+        double x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = w[k + u];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          s = s + x[u];
+          w[k + u] = s;
         }
       }
+      for (; k <= hxe; ++k) {
+        s = s + w[k];
+        w[k] = s;
+      }
+    }
+    lds_order();
+#pragma unroll
+    for (int c = 0; c < kNormC; ++c) {
+      const int q = i0 + 64 * c + lane, i = q < nx ? q : nx - 1;
+      const int e = hxe < nx - 1 - i ? hxe : nx - 1 - i, w = hxe < i ? hxe : i;
+#pragma unroll
+      for (int r = 0; r < RN; ++r)
+        if (jj >= lo[r] && jj <= hi[r])
+          den[r][c] = ((den[r][c] + wl[r * ld + e]) + wl[r * ld + w]) + w0[r];
+    }
+  }
+  __syncthreads();
+  double *out = P.den + (size_t)blockIdx.y * nx * ny;
+  for (int r = 0; r < RN; ++r) {
+    // the waves' sums of one row at a time, through LDS
+#pragma unroll
+    for (int c = 0; c < kNormC; ++c) lds[(sw * kNormC + c) * 64 + lane] = den[0][c];
+#pragma unroll
+    for (int q = 0; q + 1 < RN; ++q)
+#pragma unroll
+      for (int c = 0; c < kNormC; ++c) den[q][c] = den[q + 1][c];
+    __syncthreads();
+    for (int c = sw; c < kNormC; c += S) {
+      double b = lds[c * 64 + lane];
+      for (int q = 1; q < S; ++q) b = b + lds[(q * kNormC + c) * 64 + lane];
+      const int i = i0 + 64 * c + lane;
+      if (i < nx && j0 + r < ny) out[(size_t)(j0 + r) * nx + i] = b;
     }
     __syncthreads();
   }
-  if (i < nx) {
-    P.out[(size_t)f * nx * ny + (size_t)j0 * nx + i] = (0.0 + s0) / t0;
-    if (two) P.out[(size_t)f * nx * ny + (size_t)(j0 + 1) * nx + i] = (0.0 + s1) / t1;
+}
+
+// Numerators and quotients.  One workgroup of S waves per (2G output rows,
+// tile of C*64/G columns, field); the 64/G lanes of a group own two output
+// rows, a lane C cells of each.  For each of its window rows a wave evaluates
+// the weights of its output rows once, stages data row j' (0 outside the
+// grid), and every lane accumulates its cells (smooth_side).
+// Per offset a lane takes 2C fused multiply-adds and reads 24 bytes of LDS;
+// the form before it (a thread per column of two rows) took a product and two
+// sums a node and 1.5 LDS reads of 8 bytes.  With C = 7 and one group the
+// reads still bound it: C = 13 and two groups halve them per node.
+// MI355X, 401^2 at 0.005 degrees: smoothing of 20 kernels at sigma 0.2 8.3 ms
+// and 0.5 for the denominators, against 33.6, the metric's 20 periods 6.2 and
+// 1.5 ms against 29.9; at the 65 TFLOP/s that independent FP64 multiply-adds
+// reach they are 4.4 and 3.2 ms.  What is left is issue: the vector units are
+// busy two thirds of the cycles, a quarter of that with the weights, the
+// zeroing and adding of the sums and the staging of each row, at a clock
+// that falls to 1.85 GHz under it.  The window rows are split over waves because the widest of a
+// call's windows are 200 times the narrowest one's work: a wave doing one
+// alone ran 5 ms.
+// C is odd: lanes C doubles apart then read 32 different LDS bank pairs.
+constexpr int kPadC = 2;  // columns staged past the window on either side, in units of C
+// LDS doubles of one wave: the weights, the staged row
+size_t smooth_lds_doubles(int G, int C, int hxe) {
+  return (size_t)2 * G * (hxe + 1) + 64 / G * C + 2 * ((size_t)hxe + (size_t)kPadC * C);
+}
+template <int G, int C, bool SMALL>
+__global__ __launch_bounds__(64 * kMaxSplit, 2) void k_smooth_geo2(GeoSmooth P, int lds_wave) {
+  static_assert(C % 2 == 1 && C >= 3, "C + 2 elements are read ahead");
+  constexpr int RW = 2 * G, kLanes = 64 / G, kTile = kLanes * C;
+  extern __shared__ double lds[];
+  const int lane = threadIdx.x & 63, g = lane / kLanes;
+  const int S = blockDim.x >> 6, sw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int j0 = RW * blockIdx.x, f = P.order[blockIdx.y], i0 = kTile * blockIdx.z;
+  const int nx = P.nx, ny = P.ny;
+  const int hx = P.hx[f], hxe = hx < nx - 1 ? hx : nx - 1;
+  const int span = hxe + kPadC * C;  // staged columns i0 - span .. i0 + kTile - 1 + span
+  double *wl = lds + (size_t)sw * lds_wave, *dl = wl + (size_t)RW * (hxe + 1);
+  const double *data = P.data + (P.ndata == 1 ? 0 : (size_t)f * nx * ny);
+  const double kap = geo_kap(P.sigma[f]);
+  int n1 = ny, n2 = -1;
+  double latr[RW], cr[RW];
+#pragma unroll
+  for (int r = 0; r < RW; ++r) {
+    const int j = j0 + r < ny ? j0 + r : ny - 1, hy = P.hy[(size_t)f * ny + j];
+    n1 = j - hy < n1 ? j - hy : n1;
+    n2 = j + hy > n2 ? j + hy : n2;
+    latr[r] = P.lat[j];
+    cr[r] = cos(latr[r] * kGeoDeg2Rad);
+  }
+  n1 = n1 > 0 ? n1 : 0;
+  n2 = n2 < ny - 1 ? n2 : ny - 1;
+  // the window rows of the lane's two output rows
+  int lo[2], hi[2];
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int j = j0 + 2 * g + r, hy = j < ny ? P.hy[(size_t)f * ny + j] : 0;
+    lo[r] = j < ny ? j - hy : ny;
+    hi[r] = j < ny ? j + hy : -1;
+  }
+  for (int q = lane; q < kTile + 2 * span; q += 64) dl[q] = 0.0;
+  const int c0 = i0 - span > 0 ? i0 - span : 0;
+  const int c1 = i0 + kTile + span < nx ? i0 + kTile + span : nx;
+  const int ic = i0 + (lane % kLanes) * C;  // the lane's first cell
+  const double *dt = dl + span + (lane % kLanes) * C, *wg = wl + 2 * g;
+  double num[2][C] = {};
+  LatTerms<RW> T;
+  for (int jj = first_row(n1, sw, S); jj <= n2; jj += S) {
+    double cc[RW], sd[RW];
+    T.at(P, jj, S, lane, latr, cr, cc, sd);
+    lds_order();  // the previous row's weights and data have been read
+    for (int k = lane; k <= hxe; k += 64) {
+      const double s2 = P.s2[k];
+#pragma unroll
+      for (int r = 0; r < RW; ++r)
+        wl[k * RW + r] = geo_weight<SMALL>(__builtin_fma(s2, cc[r], sd[r]), kap);
+    }
+    const double *row = data + (size_t)jj * nx;
+    for (int q = c0 + lane; q < c1; q += 64) dl[q - i0 + span] = row[q];
+    lds_order();
+    const bool in0 = jj >= lo[0] && jj <= hi[0], in1 = jj >= lo[1] && jj <= hi[1];
+    if (in0 && in1) {
+      smooth_side<2, RW, C, 1>(wg + RW, dt + 1, hxe, num);
+      smooth_side<2, RW, C, -1>(wg + RW, dt - 1, hxe, num);
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int c = 0; c < C; ++c) num[r][c] = __builtin_fma(wg[r], dt[c], num[r][c]);
+    } else if (in0 || in1) {  // a window row of one of the two output rows
+      const double *w1 = in0 ? wg : wg + 1;
+      double one[1][C];
+#pragma unroll
+      for (int c = 0; c < C; ++c) one[0][c] = in0 ? num[0][c] : num[1][c];
+      smooth_side<1, RW, C, 1>(w1 + RW, dt + 1, hxe, one);
+      smooth_side<1, RW, C, -1>(w1 + RW, dt - 1, hxe, one);
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const double v = __builtin_fma(w1[0], dt[c], one[0][c]);
+        num[0][c] = in0 ? v : num[0][c];
+        num[1][c] = in0 ? num[1][c] : v;
+      }
+    }
+  }
+  // the waves' sums, added in wave order: [wave][2C][64] in LDS
+  __syncthreads();
+  if (sw > 0) {
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+        lds[((size_t)(sw - 1) * 2 * C + r * C + c) * 64 + lane] = num[r][c];
+  }
+  __syncthreads();
+  if (sw > 0) return;
+  double *out = P.out + (size_t)f * nx * ny;
+  const double *den = P.den + (size_t)P.norm_of[f] * nx * ny;
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int j = j0 + 2 * g + r;
+    if (j >= ny) continue;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      double a = num[r][c];
+      for (int q = 0; q < S - 1; ++q) a = a + lds[((size_t)q * 2 * C + r * C + c) * 64 + lane];
+      if (ic + c < nx) out[(size_t)j * nx + ic + c] = a / den[(size_t)j * nx + ic + c];
+    }
   }
 }
 
@@ -379,23 +509,77 @@ dim3 flat_grid(size_t n) { return dim3((unsigned)((n + 255) / 256)); }
 
 }  // namespace
 
-size_t smooth_lds_bytes(int nx) { return 2 * (size_t)nx * sizeof(double); }
-
 void launch_geo_s2(hipStream_t s, const double *lon, int nx, double *s2) {
   hipLaunchKernelGGL(k_geo_s2, flat_grid((size_t)nx), dim3(256), 0, s, lon, nx, s2);
 }
 
-void launch_smooth_geo2(hipStream_t s, const GeoSmooth &P, int nfield) {
-  const dim3 grid((unsigned)P.ny, (unsigned)nfield);
-  const size_t lds = smooth_lds_bytes(P.nx);
-  if (P.nx <= 1024) {  // one cell per thread, two output rows per workgroup
-    hipLaunchKernelGGL(k_smooth_geo2_pair, dim3((unsigned)((P.ny + 1) / 2), (unsigned)nfield),
-                       dim3((P.nx + 63) / 64 * 64), 3 * (size_t)P.nx * sizeof(double), s, P);
-  } else if (P.nx <= 2048) {
-    hipLaunchKernelGGL((k_smooth_geo2<4, 512>), grid, dim3(512), lds, s, P);
-  } else {  // nx <= 4096 (SATT_GEO_MAX_NX)
-    hipLaunchKernelGGL((k_smooth_geo2<8, 512>), grid, dim3(512), lds, s, P);
-  }
+namespace {
+
+template <int RN>
+void norm_launch(hipStream_t s, const GeoSmooth &P, int nnorm, int S) {
+  const size_t wave = (size_t)RN * ((P.hx_max + 1) | 1);
+  const size_t lds = S * std::max(wave, (size_t)64 * kNormC) * sizeof(double);
+  const dim3 grid((unsigned)((P.ny + RN - 1) / RN), (unsigned)nnorm,
+                  (unsigned)((P.nx + 64 * kNormC - 1) / (64 * kNormC)));
+  if (P.a_max <= kSmallA)
+    hipLaunchKernelGGL((k_smooth_norm<RN, true>), grid, dim3(64 * S), lds, s, P, (int)wave);
+  else
+    hipLaunchKernelGGL((k_smooth_norm<RN, false>), grid, dim3(64 * S), lds, s, P, (int)wave);
+}
+
+template <int G, int C>
+void smooth_launch(hipStream_t s, const GeoSmooth &P, int nfield, int nnorm) {
+  // the waves of a workgroup: as many as leave two workgroups a CU
+  const size_t wave = smooth_lds_doubles(G, C, P.hx_max);
+  int S = kMaxSplit;
+  while (S > 1 && S * wave * sizeof(double) > 80 * 1024) S >>= 1;
+  if (8 * S * (P.hx_max + 2) * sizeof(double) <= 80 * 1024)
+    norm_launch<8>(s, P, nnorm, S);
+  else
+    norm_launch<1>(s, P, nnorm, S);
+  const size_t sums = (size_t)(S - 1) * 2 * C * 64;
+  const size_t lds = std::max(S * wave, sums) * sizeof(double);
+  constexpr int kTile = 64 / G * C;
+  const dim3 grid((unsigned)((P.ny + 2 * G - 1) / (2 * G)), (unsigned)nfield,
+                  (unsigned)((P.nx + kTile - 1) / kTile));
+  if (P.a_max <= kSmallA)
+    hipLaunchKernelGGL((k_smooth_geo2<G, C, true>), grid, dim3(64 * S), lds, s, P, (int)wave);
+  else
+    hipLaunchKernelGGL((k_smooth_geo2<G, C, false>), grid, dim3(64 * S), lds, s, P, (int)wave);
+}
+
+}  // namespace
+
+// The tile (G lane groups, C columns a lane) whose columns cover a row with
+// the fewest idle lanes; at equal cover the wider C.  Windows whose weights
+// of 2G rows and staged row pass 64 KB take one group.
+void launch_smooth_geo2(hipStream_t s, const GeoSmooth &P, int nfield, int nnorm) {
+  int bg = 1, bc = 13, cover = INT_MAX;
+  for (int C : {13, 11, 9})
+    for (int G : {1, 2, 4}) {
+      if (G > 1 && smooth_lds_doubles(G, C, P.hx_max) * sizeof(double) > 64 * 1024) continue;
+      const int tile = 64 / G * C, n = (P.nx + tile - 1) / tile * tile;
+      if (n < cover) {
+        cover = n;
+        bg = G;
+        bc = C;
+      }
+    }
+  auto go = [&](auto c) {
+    constexpr int C = decltype(c)::value;
+    if (bg == 1)
+      smooth_launch<1, C>(s, P, nfield, nnorm);
+    else if (bg == 2)
+      smooth_launch<2, C>(s, P, nfield, nnorm);
+    else
+      smooth_launch<4, C>(s, P, nfield, nnorm);
+  };
+  if (bc == 13)
+    go(std::integral_constant<int, 13>{});
+  else if (bc == 11)
+    go(std::integral_constant<int, 11>{});
+  else
+    go(std::integral_constant<int, 9>{});
 }
 
 void launch_gradient_geo2(hipStream_t s, const GeoGrad &G, int nf, const double *f_nat,

@@ -199,6 +199,12 @@ struct GeoSmooth {
   const double *s2;             // sin((lon(k)-lon(0))*deg2rad/2)**2, k < nx
   const double *data, *sigma;
   const int *hx, *hy;
+  const int *order;             // the fields, widest window first
+  const int *norm_of;           // each field's distinct sigma
+  const int *norm_field;        // a field of each distinct sigma, widest first
+  double *den;                  // [distinct sigma][j][i]: the weights' sums
+  int hx_max;                   // widest half-width, at most nx - 1
+  double a_max;                 // bound on sin(theta/2)**2 over every window
   double *out;                  // [f][j][i]
 };
 struct GeoGrad {
@@ -206,9 +212,8 @@ struct GeoGrad {
   const double *lon, *lat;      // degrees
   const double *cosd_lat;       // cosd(lat(j)), host-computed
 };
-size_t smooth_lds_bytes(int nx);
 void launch_geo_s2(hipStream_t s, const double *lon, int nx, double *s2);
-void launch_smooth_geo2(hipStream_t s, const GeoSmooth &P, int nfield);
+void launch_smooth_geo2(hipStream_t s, const GeoSmooth &P, int nfield, int nnorm);
 // tx, ty period-major (nf, nx, ny) of nf natural fields
 void launch_gradient_geo2(hipStream_t s, const GeoGrad &G, int nf, const double *f_nat,
                           double *tx_pm, double *ty_pm);

@@ -72,6 +72,40 @@ def test_smoothing_is_deterministic_and_keeps_constants(ctx):
     assert np.all(ctx.smooth_geo2(lons, lats, np.ones((50, 40)), 0.07) == 1.0)
 
 
+@pytest.mark.parametrize("nx,ny,d,sigmas", [
+    (2, 2, 0.05, [0.02, 0.3]),            # the smallest grid
+    (144, 5, 0.02, [0.03, 0.1, 0.03]),    # four lane groups, a full tile; two fields of one sigma
+    (145, 9, 0.02, [0.05]),               # one column past it
+    (416, 6, 0.005, [0.05, 0.2]),         # two groups, a full tile, rows a multiple of neither
+    (417, 3, 0.005, [0.02]),
+    (833, 3, 0.002, [0.3]),               # one group, two tiles, windows wider than the grid
+    (2600, 2, 0.001, [2.0]),              # the weights leave one wave a workgroup
+    (40, 12, 1.5, [6.0, 9.0]),            # distances past the series of asin^2
+])
+def test_smoothing_tiles_match_oracle(ctx, nx, ny, d, sigmas):
+    """Same tolerance as above: every node's weight is within a few ulp, and
+    the sums' rounding is far below it."""
+    lons, lats = axes(nx, ny, d)
+    data = field(nx, ny, 3 * nx + ny, len(sigmas))
+    out = ctx.smooth_geo2(lons, lats, data, sigmas).reshape(data.shape)
+    for f, s in enumerate(sigmas):
+        smooth_close(out[f], O.smooth_geo2(lons, lats, data[f], s), data[f])
+    ones = ctx.smooth_geo2(lons, lats, np.ones((nx, ny)), sigmas)
+    assert np.all(ones == 1.0)
+
+
+def test_smoothing_keeps_nan_and_infinity_in_their_windows(ctx):
+    lons, lats = axes(150, 37, 0.02)
+    z = field(150, 37, 11)
+    z[71, 20], z[3, 4] = np.nan, np.inf
+    got, want = ctx.smooth_geo2(lons, lats, z, 0.06), O.smooth_geo2(lons, lats, z, 0.06)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isinf(got), np.isinf(want))
+    fine = np.isfinite(want)
+    assert fine.any() and not fine.all()
+    smooth_close(got[fine], want[fine], z[np.isfinite(z)])
+
+
 def test_gradient_bitwise(ctx):
     lons, lats = axes(33, 27, 0.04, 95.0, -10.0)
     f = field(33, 27, 3, 3)
