@@ -64,6 +64,7 @@
 #include <climits>
 #include <type_traits>
 
+#include "satt_div.h"
 #include "satt_internal.h"
 #include "satt_strip.h"
 
@@ -164,84 +165,133 @@ __device__ __forceinline__ double own_reg(double x) {
   return y;
 }
 
-// One cell of the forward sweep body (src/eikon_solver_2d.f90:910-1079) with
-// every operand in registers.  Every floating-point expression is the
-// reference's, in its order; what the four quadrants have in common is
-// evaluated once: px, qx and the a-terms depend only on the x neighbour (W or
-// E), py, qy and the b-terms only on the y neighbour (S or N), so e.g.
+// One cell of the forward sweep body (src/eikon_solver_2d.f90:910-1079) in
+// the sweep direction (XD, YD), every operand in registers.  tau becomes the
+// least of itself and the accepted candidates, so a candidate that cannot be
+// accepted, or that an earlier evaluation has already taken, need not be
+// evaluated; every value that is taken comes from the reference's
+// expressions, in their order, with what the quadrants have in common
+// evaluated once: px, qx and the a-terms depend only on the x neighbour, py,
+// qy and the b-terms only on the y neighbour, so e.g.
 // ak*(px*px) + bk*(py*py) - 2*ck*px*py is (A1x + B1y) - C1x*py with the same
-// operands and roundings.  Quadrants and one-sided candidates at the grid
-// boundary, which the reference skips, are evaluated and discarded.
-// dis_x = sqrt(fun**2*(b/(a*b-c**2))) and dis_y = sqrt(fun**2*(a/(a*b-c**2)))
-// are per-cell constants precomputed by the same expression.
-__device__ __forceinline__ double fwd_cell_r(int i, int j, int nx, int ny, double dx, double dy,
-                                             double ak, double bk, double ck, double fk,
-                                             double disx, double disy, double t0, double t0x,
-                                             double t0y, double tc, double tW, double tE,
-                                             double tS, double tN, double zW, double zE,
-                                             double zS, double zN) {
-  const double t0dx = t0 / dx, t0dy = t0 / dy;
-  // x neighbour: 0 = W (i-1), 1 = E (i+1); y neighbour: 0 = S (j-1), 1 = N (j+1)
-  const double px[2] = {t0x + t0dx, t0x - t0dx};
-  const double qx[2] = {-(t0dx * tW), t0dx * tE};
-  const double py[2] = {t0y + t0dy, t0y - t0dy};
-  const double qy[2] = {-(t0dy * tS), t0dy * tN};
-  const bool hx[2] = {i > 0, i < nx - 1};
-  const bool hy[2] = {j > 0, j < ny - 1};
+// operands and roundings.  Index 0 is the upwind neighbour of the sweep, 1
+// the downwind one.  dis_x = sqrt(fun**2*(b/(a*b-c**2))) and dis_y =
+// sqrt(fun**2*(a/(a*b-c**2))) are per-cell constants precomputed by the same
+// expression.  What is left out:
+//  - Candidates whose neighbours have not changed since the cell was last
+//    evaluated.  A downwind neighbour that was upwind in the sweep before had
+//    been updated there before the cell was: in the reference's order of
+//    sweeps that is the downwind y neighbour of every sweep and the downwind
+//    x neighbour where YD > 0.  FIRST (the first sweep of a solve) has none.
+//  - Roots that fail the tests by more than rounding can move them.  With
+//    chx, chy the tested components, px*chx + py*chy = ea*t + eb/2 at any t,
+//    which at the lesser root is -sqrt(delta)/2: where px and py have their
+//    neighbours' signs, chx and chy cannot both have them there.  And the
+//    greater root cannot lie below tau where 2 ea tau + eb < sqrt(delta).
+//    Both need ea > 0 and delta above 1e-12 eb^2: a root of delta is then
+//    1e-6 |eb| or more, against rounding of about 1e-15 |eb| in these
+//    terms; the second has a margin of 1e-6 beside.  A comparison with NaN
+//    is false, and the roots are evaluated.
+//  - The greater one-sided value where it exceeds tau, and the lesser where
+//    its time falls short of the neighbour's, by more than 1e-12 of them.
+// One cell took 18 divisions and 4 square roots, 2100 cycles of a SIMD; in
+// the later iterations most waves now take the roots of one or two quadrants
+// and no one-sided value: about 350 instructions a step against 630.  MI355X,
+// forward sweeps: 600 solves at 401^2 99.8 -> 56 ms, 1600 at 41^2 4.8 -> 3.2 ms.
+template <int XD, int YD, bool FIRST>
+__device__ __forceinline__ double fwd_cell_r(int i, int j, int nx, int ny, const Recip &rdx,
+                                             const Recip &rdy, double ak, double bk, double ck,
+                                             double fk, double disx, double disy, double t0,
+                                             double t0x, double t0y, double tc,
+                                             const double (&tx)[2], const double (&ty)[2],
+                                             const double (&zx)[2], const double (&zy)[2]) {
+  constexpr bool kNewX = FIRST || YD < 0;  // the downwind x neighbour may have changed
+  const double t0dx = quot(t0, rdx), t0dy = quot(t0, rdy);
+  constexpr int sx[2] = {XD, -XD}, sy[2] = {YD, -YD};  // +1: W or S, -1: E or N
+  double px[2], qx[2], py[2], qy[2];
+  bool hx[2], hy[2];
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+    px[n] = sx[n] > 0 ? t0x + t0dx : t0x - t0dx;
+    qx[n] = sx[n] > 0 ? -(t0dx * tx[n]) : t0dx * tx[n];
+    py[n] = sy[n] > 0 ? t0y + t0dy : t0y - t0dy;
+    qy[n] = sy[n] > 0 ? -(t0dy * ty[n]) : t0dy * ty[n];
+    hx[n] = sx[n] > 0 ? i > 0 : i < nx - 1;
+    hy[n] = sy[n] > 0 ? j > 0 : j < ny - 1;
+  }
   const double ak2 = 2 * ak, bk2 = 2 * bk, ck2 = 2 * ck, ff = fk * fk;
   double A1[2], A2[2], A3[2], C1[2], C2[2], B1[2], B2[2], B3[2];
 #pragma unroll
-  for (int x = 0; x < 2; ++x) {
-    A1[x] = ak * (px[x] * px[x]);
-    A2[x] = ak2 * px[x] * qx[x];
-    A3[x] = ak * (qx[x] * qx[x]);
-    C1[x] = ck2 * px[x];
-    C2[x] = ck2 * qx[x];
-  }
-#pragma unroll
-  for (int y = 0; y < 2; ++y) {
-    B1[y] = bk * (py[y] * py[y]);
-    B2[y] = bk2 * py[y] * qy[y];
-    B3[y] = bk * (qy[y] * qy[y]);
+  for (int n = 0; n < 2; ++n) {
+    A1[n] = ak * (px[n] * px[n]);
+    A2[n] = ak2 * px[n] * qx[n];
+    A3[n] = ak * (qx[n] * qx[n]);
+    C1[n] = ck2 * px[n];
+    C2[n] = ck2 * qx[n];
+    B1[n] = bk * (py[n] * py[n]);
+    B2[n] = bk2 * py[n] * qy[n];
+    B3[n] = bk * (qy[n] * qy[n]);
   }
   double tnew = tc;
-  // quadrants in the reference's order: (W,S), (W,N), (E,S), (E,N); the
-  // causality test requires chx >= 0 with W, <= 0 with E, chy >= 0 with S,
-  // <= 0 with N
+  // the causality test requires chx >= 0 with W, <= 0 with E, chy >= 0 with
+  // S, <= 0 with N
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int x = q >> 1, y = q & 1;
+    if (x && y && !kNewX) continue;
     const double ea = A1[x] + B1[y] - C1[x] * py[y];
     const double eb = A2[x] + B2[y] - ck2 * (px[x] * qy[y] + py[y] * qx[x]);
     const double ec = A3[x] + B3[y] - C2[x] * qy[y] - ff;
-    const double delta = eb * eb - 4 * ea * ec;
-    const bool use = hx[x] && hy[y] && delta >= 0;
-    const double sq = sqrt(delta);
-#pragma unroll
-    for (int isol = 1; isol <= 2; ++isol) {
-      const double tt = isol == 1 ? (-eb + sq) / (2 * ea) : (-eb - sq) / (2 * ea);
-      const double Tx = px[x] * tt + qx[x];
-      const double Ty = py[y] * tt + qy[y];
-      const double chx = ak * Tx - ck * Ty;
-      const double chy = bk * Ty - ck * Tx;
-      const bool ok = (x == 0 ? chx >= 0 : chx <= 0) && (y == 0 ? chy >= 0 : chy <= 0);
-      if (use && ok && tt < tnew) tnew = tt;
+    const double ebb = eb * eb;
+    const double delta = ebb - 4 * ea * ec;
+    const double ea2 = 2 * ea;
+    const bool one = ea > 0 && (sx[x] > 0 ? px[x] > 0 : px[x] < 0) &&
+                     (sy[y] > 0 ? py[y] > 0 : py[y] < 0) && delta > 1e-12 * ebb;
+    const double h = __builtin_fma(ea2, tnew, eb);
+    const bool above = h < 0 || h * h < (1 - 1e-6) * delta;  // the greater root is above tau
+    if (hx[x] && hy[y] && delta >= 0 && !(one && above)) {
+      const double sq = root_of(delta);
+      const Recip re = recip_of(ea2);
+      auto take = [&](double tt) {
+        const double Tx = px[x] * tt + qx[x];
+        const double Ty = py[y] * tt + qy[y];
+        const double chx = ak * Tx - ck * Ty;
+        const double chy = bk * Ty - ck * Tx;
+        const bool ok = (sx[x] > 0 ? chx >= 0 : chx <= 0) && (sy[y] > 0 ? chy >= 0 : chy <= 0);
+        if (ok && tt < tnew) tnew = tt;
+      };
+      take(quot(-eb + sq, re));
+      if (!one) take(quot(-eb - sq, re));
     }
   }
-  // one-sided candidates (:996-1075): W, E, S, N
+  // one-sided candidates (:996-1075), the roots of p*tt + q = +-dis: with P =
+  // p and Q = -q for W and S, P = -p and Q = q for E and N, (Q + dis)/P and
+  // (Q - dis)/P
 #pragma unroll
   for (int n = 0; n < 4; ++n) {
     const bool isx = n < 2;
     const int s = n & 1;
+    if (s && !(isx ? kNewX : FIRST)) continue;
+    const int sg = isx ? sx[s] : sy[s];
     const double p = isx ? px[s] : py[s], q = isx ? qx[s] : qy[s];
+    const double P = sg > 0 ? p : -p, Q = sg > 0 ? -q : q;
     const double dis = isx ? disx : disy;
-    const double tn = n == 0 ? tW : n == 1 ? tE : n == 2 ? tS : tN;
-    const double t0n = n == 0 ? zW : n == 1 ? zE : n == 2 ? zS : zN;
+    const double tn = isx ? tx[s] : ty[s], t0n = isx ? zx[s] : zy[s];
     const bool use = isx ? hx[s] : hy[s];
-    double tt = (dis - q) / p;
-    if (use && tt * t0 >= tn * t0n && tt > tn * 0.5 && tt < tnew) tnew = tt;
-    tt = (-dis - q) / p;
-    if (use && tt * t0 >= tn * t0n && tt > tn * 0.5 && tt < tnew) tnew = tt;
+    const double up = Q + dis, dn = Q - dis, Tn = tn * t0n;
+    // with P > 0, the greater value above tau and the lesser one's time short
+    // of the neighbour's
+    const double dt = dn * t0;
+    const bool none = P > 0 && __builtin_fma(-tnew, P, up) > 1e-12 * fabs(up) &&
+                      __builtin_fma(Tn, P, -dt) > 1e-12 * fabs(dt);
+    if (use && !none) {
+      const Recip rp = recip_of(P);
+      const double lim = tn * 0.5;
+      double tt = quot(up, rp);
+      if (tt * t0 >= Tn && tt > lim && tt < tnew) tnew = tt;
+      tt = quot(dn, rp);
+      if (tt * t0 >= Tn && tt > lim && tt < tnew) tnew = tt;
+    }
   }
   return tnew;
 }
@@ -666,7 +716,7 @@ __device__ __forceinline__ float as_f(unsigned u) { return __builtin_bit_cast(fl
 #define SATT_COPY_KU_F64 8
 #endif
 template <typename V, int FROM>
-__device__ void skew_copy(const Team &T, const GMEM V *__restrict__ src, GMEM V *__restrict__ dst, int nx,
+__device__ __forceinline__ void skew_copy(const Team &T, const GMEM V *__restrict__ src, GMEM V *__restrict__ dst, int nx,
                           int ny, int R, int ns, int lane) {
   constexpr int TO = 1 - FROM;
   constexpr int kU = sizeof(V) == 4 ? SATT_COPY_KU_F32 : SATT_COPY_KU_F64;
@@ -759,7 +809,7 @@ template <typename V>
 struct FwdCtx {
   int nx, ny, R, lane;
   size_t SE;
-  double dx, dy;           // FP64 update
+  Recip dx, dy;            // the full update
   V rdx, rdy;              // upwind update: 1/dx, 1/dy in V
   int fi0, fi1, fj0, fj1;  // frozen rectangle
   // period skews (plus, minus), kPF fields each, and item T0 skews (plus,
@@ -778,11 +828,12 @@ struct FwdCtx {
 // One sweep (XD, YD) over the k-th strip of the sweep, updating tau in place
 // in the sweep's own skew: the reference's update (UP false, FP64) or the
 // mixed mode's upwind update on dtau (UP true).  MODE 0: plain; 1: record
-// the snapshot (first sweep of an iteration); 2: the strip's sum and max of
+// the snapshot (first sweep of an iteration); 3: the same in the first
+// iteration of the full update (fwd_cell_r's FIRST); 2: the strip's sum and max of
 // |tau-snap|*T0 in double (last sweep) into ss, sm.  PD: how many steps
 // ahead the operands are fetched.
 template <typename V, int XD, int YD, int MODE, bool UP, int PD>
-__device__ void fwd_strip_pass(const FwdCtx<V> &C, const Team &T, int k, GMEM V *tau, double &ss,
+__device__ __forceinline__ void fwd_strip_pass(const FwdCtx<V> &C, const Team &T, int k, GMEM V *tau, double &ss,
                                double &sm) {
   constexpr int SK = XD == YD ? 0 : 1;
   const int nx = C.nx, ny = C.ny, R = C.R, lane = C.lane;
@@ -828,7 +879,10 @@ __device__ void fwd_strip_pass(const FwdCtx<V> &C, const Team &T, int k, GMEM V 
   // behind a branch: a load that a branch may skip leaves the compiler
   // unsure how many loads are in flight, and it then waits for all of them,
   // the prefetched ones included.
-  // The far and near operands of step t (both fetched PD steps ahead).
+  // The far and near operands of step t (both fetched PD steps ahead; the
+  // full update's near ones one step ahead, at the position e1 of step t - PD
+  // + 1, which saves a set of registers and with it a wave per SIMD).
+  size_t e1 = 0;
   auto load_ops = [&](int t, FFar<V> &q, FNear<PS> &n) {
     const int u = t - lag;
     const int j = YD > 0 ? u : ny - 1 - u;
@@ -847,10 +901,11 @@ __device__ void fwd_strip_pass(const FwdCtx<V> &C, const Team &T, int k, GMEM V 
       else
         q.t0 = fis.ldn(0, e);  // the polish's FP64 T0
     } else {
+      n.a = fps.ld(0, e1); n.b = fps.ld(1, e1); n.c = fps.ld(2, e1); n.f = fps.ld(3, e1);
+      n.dx_ = fps.ld(4, e1); n.dy_ = fps.ld(5, e1);
+      n.t0x = fgs.ld(1, e1); n.t0y = fgs.ld(2, e1);
       q.t0 = fis.ld(0, e);
-      n.a = fps.ld(0, e); n.b = fps.ld(1, e); n.c = fps.ld(2, e); n.f = fps.ld(3, e);
-      n.dx_ = fps.ld(4, e); n.dy_ = fps.ld(5, e);
-      n.t0x = fgs.ld(1, e); n.t0y = fgs.ld(2, e);
+      e1 = e;
     }
     if constexpr (kF) {
       q.tau = ftau.ldn(0, e);
@@ -897,7 +952,8 @@ __device__ void fwd_strip_pass(const FwdCtx<V> &C, const Team &T, int k, GMEM V 
   FNear<PS> ns[S] = {};
   V tprev = 0, zprev = 0;  // own result and T0 of the previous step
   auto step = [&](int t, const FFar<V> &fc, const FFar<V> &fn, FFar<V> &f2,
-                  const FNear<PS> &nc, FNear<PS> &nx2, int tnear) {
+                  const FNear<PS> &nc, FNear<PS> &nx2,
+                  int tnear) __attribute__((always_inline)) {
     V tU = 0, zU = 0;
     load_up(t, fc.act, tU, zU);
     load_ops(t + PD, f2, nx2);
@@ -917,13 +973,12 @@ __device__ void fwd_strip_pass(const FwdCtx<V> &C, const Team &T, int k, GMEM V 
     if (fc.act) {
       const bool frozen = i >= C.fi0 && i <= C.fi1 && jc >= C.fj0 && jc <= C.fj1;
       if constexpr (kDown) {
-        const V tW = XD > 0 ? tUx : tDx, tE = XD > 0 ? tDx : tUx;
-        const V zW = XD > 0 ? zUx : zDx, zE = XD > 0 ? zDx : zUx;
-        const V tS = YD > 0 ? tprev : fn.tau, tN = YD > 0 ? fn.tau : tprev;
-        const V zS = YD > 0 ? zprev : fn.t0, zN = YD > 0 ? fn.t0 : zprev;
+        const V tx[2] = {tUx, tDx}, ty[2] = {tprev, fn.tau};
+        const V zx[2] = {zUx, zDx}, zy[2] = {zprev, fn.t0};
         if (!frozen)
-          tnew = fwd_cell_r(i, jc, nx, ny, C.dx, C.dy, nc.a, nc.b, nc.c, nc.f, nc.dx_, nc.dy_,
-                            fc.t0, nc.t0x, nc.t0y, fc.tau, tW, tE, tS, tN, zW, zE, zS, zN);
+          tnew = fwd_cell_r<XD, YD, MODE == 3>(i, jc, nx, ny, C.dx, C.dy, nc.a, nc.b, nc.c, nc.f,
+                                               nc.dx_, nc.dy_, fc.t0, nc.t0x, nc.t0y, fc.tau, tx,
+                                               ty, zx, zy);
       } else {
         if (!frozen)
           tnew = fwd_cell_up_r<V, XD, YD>(i, jc, nx, ny, C.rdx, C.rdy, (V)nc.a, (V)nc.b, (V)nc.c,
@@ -936,7 +991,7 @@ __device__ void fwd_strip_pass(const FwdCtx<V> &C, const Team &T, int k, GMEM V 
         if (MODE == 1) fsnap.stn(0, e, fc.tau);
       } else {
         ftau.st(0, e, tnew);
-        if (MODE == 1) fsnap.st(0, e, fc.tau);
+        if (MODE == 1 || MODE == 3) fsnap.st(0, e, fc.tau);
       }
       if (pub) team_publish2<V>(T, t - lag, tnew, fc.t0, base_out + t - lag + 1);
       if (MODE == 2) {
@@ -957,7 +1012,8 @@ __device__ void fwd_strip_pass(const FwdCtx<V> &C, const Team &T, int k, GMEM V 
   for (int t = -PD; t < nsteps; t += S) {
 #pragma unroll
     for (int q = 0; q < S; ++q)
-      step(t + q, fs[q], fs[(q + 1) % S], fs[(q + PD) % S], ns[q], ns[(q + PD) % S], t + q + PD);
+      step(t + q, fs[q], fs[(q + 1) % S], fs[(q + PD) % S], ns[q], ns[(q + (UP ? PD : 1)) % S],
+           t + q + PD);
   }
   if (MODE == 2) {
     ss = wave_sum(acc_s);
@@ -967,7 +1023,7 @@ __device__ void fwd_strip_pass(const FwdCtx<V> &C, const Team &T, int k, GMEM V 
 }
 
 template <typename V, int XD, int YD, int MODE, bool UP, int PD>
-__device__ void fwd_sweep(const FwdCtx<V> &C, Team &T, GMEM V *tau, StripAcc &acc) {
+__device__ __forceinline__ void fwd_sweep(const FwdCtx<V> &C, Team &T, GMEM V *tau, StripAcc &acc) {
   team_sweep_begin(T);
   for (int k = T.w; k < T.ns; k += T.W) {
     double ss = 0, sm = 0;
@@ -983,9 +1039,13 @@ __device__ void fwd_sweep(const FwdCtx<V> &C, Team &T, GMEM V *tau, StripAcc &ac
 // last in the plus skew, with the field copied between the skews at the
 // two family changes.  Returns whether the stop rule (:1091-1115) holds.
 template <typename V, bool UP, int PD>
-__device__ bool fwd_iteration(const FwdCtx<V> &C, Team &T, GMEM V *tP, GMEM V *tM) {
+__device__ __forceinline__ bool fwd_iteration(const FwdCtx<V> &C, Team &T, GMEM V *tP, GMEM V *tM,
+                              bool first = false) {
   StripAcc acc;
-  fwd_sweep<V, 1, 1, 1, UP, PD>(C, T, tP, acc);
+  if (!UP && first)
+    fwd_sweep<V, 1, 1, UP ? 1 : 3, UP, PD>(C, T, tP, acc);
+  else
+    fwd_sweep<V, 1, 1, 1, UP, PD>(C, T, tP, acc);
   skew_copy<V, 0>(T, tP, tM, C.nx, C.ny, C.R, T.ns, C.lane);
   fwd_sweep<V, 1, -1, 0, UP, PD>(C, T, tM, acc);
   fwd_sweep<V, -1, 1, 0, UP, PD>(C, T, tM, acc);
@@ -1169,7 +1229,7 @@ template <typename V>
 __device__ void fwd_ctx_init(FwdCtx<V> &C, const Grid &g, const SkewGeom &sg, int lane,
                              const int rect[4]) {
   C.nx = g.nx; C.ny = g.ny; C.R = sg.R; C.lane = lane; C.SE = sg.skew_elems();
-  C.dx = g.dx; C.dy = g.dy;
+  C.dx = recip_of(g.dx); C.dy = recip_of(g.dy);
   C.rdx = (V)(1.0 / g.dx); C.rdy = (V)(1.0 / g.dy);
   C.fi0 = rect[0]; C.fi1 = rect[1]; C.fj0 = rect[2]; C.fj1 = rect[3];
 }
@@ -1179,7 +1239,7 @@ __device__ void fwd_ctx_init(FwdCtx<V> &C, const Grid &g, const SkewGeom &sg, in
 // layout: the reference's update on tau (UP false), or the mixed mode's
 // upwind update on dtau, with T = (1 + dtau)*T0 (UP true).
 template <bool UP, int PD>
-__device__ void fwd_finish64(const SlotDesc &D, Team &T, int lane, const int rect[4]) {
+__device__ __forceinline__ void fwd_finish64(const SlotDesc &D, Team &T, int lane, const int rect[4]) {
   const Grid &g = D.g;
   const SkewGeom &sg = D.sg;
   const int nx = g.nx, ny = g.ny, R = sg.R, ns = sg.ns;
@@ -1210,7 +1270,7 @@ __device__ void fwd_finish64(const SlotDesc &D, Team &T, int lane, const int rec
   int iter = 1;
   bool conv = false;
   for (; iter <= kFwdMaxIter; ++iter)
-    if (fwd_iteration<double, UP, PD>(C, T, gm(tauP), gm(tauM))) { conv = true; break; }
+    if (fwd_iteration<double, UP, PD>(C, T, gm(tauP), gm(tauM), iter == 1)) { conv = true; break; }
   if (!conv) iter = kFwdMaxIter;
   auto tau_of = [&](double v) { return UP ? 1.0 + v : v; };
   const GMEM double *gtau = gm(tauP);
@@ -1247,8 +1307,11 @@ __device__ bool fwd_item_rect(const SlotDesc &D, int lane, int rect[4]) {
 // The strip kernels run one item per workgroup of W = blockDim.x/64 waves
 // (a team), with team_lds_bytes of dynamic LDS when W > 1, fetching the
 // sweeps' operands PD steps ahead.
+// Held to three waves per SIMD (168 registers, some fifteen of them spilled):
+// 600 solves at 401^2 56.0 ms against 69.4 with the 184 registers that two
+// waves may have, 1600 solves at 41^2 3.19 against 3.12.
 template <bool TEAM, int PD>
-__global__ __launch_bounds__(TEAM ? 64 * kMaxTeam : 64) void k_fwd_strip(const SlotDesc *sd) {
+__global__ __launch_bounds__(TEAM ? 64 * kMaxTeam : 64, 3) void k_fwd_strip(const SlotDesc *sd) {
   extern __shared__ double lds[];
   const SlotDesc D = sd[blockIdx.x];
   const int lane = threadIdx.x & 63;

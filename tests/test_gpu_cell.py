@@ -1,0 +1,62 @@
+"""The batched FP64 sweeps, whose cell leaves out candidates that cannot be
+accepted, against the one-solve-per-launch kernels, which evaluate every
+candidate of the reference's update: the same bits and iteration counts, where
+a candidate is left out by the narrowest margins or may not be left out."""
+import numpy as np
+import pytest
+
+import satt
+import satt_workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def model(kind, nx, ny, rng):
+    """(velocity, m11, m12, m22)"""
+    one, zero = np.ones((nx, ny)), np.zeros((nx, ny))
+    if kind == "ties":          # every quadrant's gradient equal: roots on the current value
+        return 3.0 * one, one, zero, one
+    if kind == "rough":         # large jumps from cell to cell
+        return np.exp(rng.uniform(np.log(0.8), np.log(8.0), (nx, ny))), one, zero, one
+    if kind == "sheared":       # m12^2 within 2% of m11 m22, of either sign
+        a, b = rng.uniform(0.5, 1, (nx, ny)), rng.uniform(0.5, 1, (nx, ny))
+        return rng.uniform(2, 4, (nx, ny)), a, 0.99 * np.sqrt(a * b) * np.sign(rng.uniform(-1, 1, (nx, ny))), b
+    if kind == "indefinite":    # no metric at all: ea of either sign in some cells
+        return rng.uniform(2, 4, (nx, ny)), one, np.where(rng.uniform(size=(nx, ny)) < 0.1, 1.2, 0.1), one
+    if kind == "nan":
+        v = rng.uniform(2, 4, (nx, ny))
+        v[rng.integers(0, nx, 3), rng.integers(0, ny, 3)] = np.nan
+        return v, one, zero, one
+    return W.smooth_random_field(nx, ny, 5.0, rng, 2.5, 4.2), one, zero, one
+
+
+@pytest.mark.parametrize("kind,nx,ny,d,lat", [
+    ("ties", 41, 37, 0.05, 20.0), ("ties", 130, 20, 0.01, -1.0), ("smooth", 65, 64, 0.02, 60.0),
+    ("smooth", 5, 70, 0.1, 0.0), ("smooth", 129, 6, 0.01, 10.0), ("rough", 64, 40, 0.01, 30.0),
+    ("rough", 90, 35, 0.5, 40.0), ("sheared", 50, 66, 0.02, 20.0), ("sheared", 67, 31, 0.02, 20.0),
+    ("indefinite", 40, 33, 0.02, 20.0), ("nan", 33, 40, 0.02, 20.0),
+])
+@pytest.mark.parametrize("waves", [1, 3])
+def test_sweeps_equal_the_full_update(ctx, kind, nx, ny, d, lat, waves):
+    rng = np.random.default_rng(nx * 1000 + ny)
+    xg, yg = 100.0 + d * np.arange(nx), lat + d * np.arange(ny)
+    v, m11, m12, m22 = model(kind, nx, ny, rng)
+    b = W.random_receiver_batch(xg, yg, v, 4, rng, nrec=(1, 9), m11=m11, m12=m12, m22=m22)
+    # one source on a node (T0 = 0 there), one on a grid line, two between nodes
+    b["item_srcx"][0], b["item_srcy"][0] = xg[nx // 2], yg[ny // 2]
+    b["item_srcx"][1] = xg[2]
+    with ctx.plan(b) as p:
+        p.set_waves(waves)
+        out, T = [], []
+        for launch in (satt.LAUNCH_BATCHED, satt.LAUNCH_PER_SOLVE):
+            p.run(True, kind != "nan", launch)
+            out.append(p.results())
+            T.append([p.item_field(k) for k in range(4)] if launch == satt.LAUNCH_BATCHED else None)
+    for k in ("iters", "tt_fwd", "chi", "item_status"):
+        np.testing.assert_array_equal(out[0][k], out[1][k], err_msg=k)
+    if kind != "nan":
+        np.testing.assert_array_equal(out[0]["adj_s"], out[1]["adj_s"])
+    for k in range(4):
+        Tk, it, _ = ctx.fwd(xg, yg, m11, m22, -m12, 1.0 / v, b["item_srcx"][k], b["item_srcy"][k])
+        np.testing.assert_array_equal(T[0][k], Tk)
+        assert it == out[0]["iters"][k, 0]
