@@ -74,6 +74,10 @@ struct satt_ctx {
   // a call whose batch differs only in the model refreshes it in place
   satt_plan *fs_plan = nullptr;
   FsKey fs_key;
+  // scratch of the per-solve entry points, kept between calls up to
+  // kSolveKeepBytes and given back with the context
+  void *solve_ws = nullptr;
+  size_t solve_ws_bytes = 0;
 };
 
 bool satt::ctx_tune_lookup(satt_ctx *ctx, const TuneKey &k, TuneWaves &out) {
@@ -245,6 +249,7 @@ extern "C" void satt_destroy(satt_ctx *ctx) {
   if (!ctx) return;
   satt_forward_simulate_release(ctx);
   (void)hipSetDevice(ctx->device);
+  if (ctx->solve_ws) (void)hipFree(ctx->solve_ws);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
 }
@@ -290,14 +295,164 @@ bool bad_fields(int nx, int ny, const void *a, const void *b, const void *c) {
 
 }  // namespace
 
-extern "C" int satt_fwd_lonlat(satt_ctx *ctx, const double *xx_deg, const double *yy_deg,
-                               int nx, int ny, const double *spha, const double *sphb,
-                               const double *sphc, const double *fun, double x0_deg,
-                               double y0_deg, double *T, int *iters) {
-  if (!ctx) return SATT_E_ARG;
-  if (bad_fields(nx, ny, spha, sphb, sphc) || !fun || !T)
-    return fail(ctx, SATT_E_ARG, "satt_fwd_lonlat: bad arguments");
-  HIPCHK(ctx, hipSetDevice(ctx->device));
+namespace {
+
+// One forward or adjoint solve on the batched sweeps: a launch group of one
+// slot whose team takes every strip of the grid it can.  The same bits as
+// the one-workgroup kernels (k_forward, k_adjoint), which step a barrier per
+// anti-diagonal on natural-layout fields; MI355X, forward and adjoint call
+// after another: 41^2 4.3 -> 2.5 ms, 401 x 343 101 -> 34.6 ms (device: forward
+// 74 -> 24.4, adjoint 25.9 -> 8.7), bound by the latency of a team's steps.
+// Grids past SATT_MAX_NY rows, and those whose skewed fields do not fit the
+// device, take those kernels.
+constexpr size_t kSolveKeepBytes = (size_t)256 << 20;
+
+// Pieces of the per-solve scratch, each on a 256-byte boundary.
+struct Carver {
+  size_t at = 0;
+  size_t take(size_t bytes) {
+    const size_t o = at;
+    at = (at + bytes + 255) & ~(size_t)255;
+    return o;
+  }
+};
+
+// The context's per-solve scratch at `bytes` or more, or null.
+char *solve_scratch(satt_ctx *ctx, size_t bytes) {
+  if (ctx->solve_ws_bytes >= bytes) return static_cast<char *>(ctx->solve_ws);
+  if (ctx->solve_ws) (void)hipFree(ctx->solve_ws);
+  ctx->solve_ws = nullptr;
+  ctx->solve_ws_bytes = 0;
+  if (hipMalloc(&ctx->solve_ws, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    ctx->solve_ws = nullptr;
+    return nullptr;
+  }
+  ctx->solve_ws_bytes = bytes;
+  return static_cast<char *>(ctx->solve_ws);
+}
+struct SolveScratchEnd {  // gives back a scratch too large to keep
+  satt_ctx *ctx;
+  ~SolveScratchEnd() {
+    if (ctx->solve_ws_bytes <= kSolveKeepBytes) return;
+    (void)hipFree(ctx->solve_ws);
+    ctx->solve_ws = nullptr;
+    ctx->solve_ws_bytes = 0;
+  }
+};
+
+// What one solve uploads at once: the item's record and its axes (degrees
+// and, by the reference's xx_deg/180.0*pi, radians), then the receivers.
+struct SolveItem {
+  SlotDesc desc;
+  int status, iters[6];
+};
+
+// The solve's descriptor, axes and receivers (rec: 3*nr values, or null) on
+// the device, the metric and the period's skewed fields; status SATT_OK, an
+// error, or 1 where the scratch does not fit the device.
+struct StripSolve {
+  GroupDims gd{};
+  SlotDesc D{}, *desc = nullptr;
+  int *status = nullptr;  // and the item's iteration counts behind it
+};
+
+int strip_solve_setup(satt_ctx *ctx, StripSolve &S, const double *xd, const double *yd, int nx,
+                      int ny, const double *spha, const double *sphb, const double *sphc,
+                      const double *fun, double x0, double y0, int nr, const double *xr,
+                      const double *yr, const double *rhs) {
+  if (!xd || !yd) return fail(ctx, SATT_E_ARG, "bad grid axes");
+  const size_t N = (size_t)nx * ny, nax = 2 * ((size_t)nx + ny);
+  const SkewGeom sg = make_skew_geom(nx, ny);
+  const size_t SE = sg.skew_elems();
+  Carver c;
+  const size_t o_item = c.take(sizeof(SolveItem) + (nax + 3 * (size_t)nr) * 8);
+  const size_t o_trig = c.take(2 * (size_t)ny * 8), o_in = c.take(4 * N * 8);
+  const size_t o_abc = c.take(3 * N * 8), o_ps = c.take(2 * (size_t)kPF * SE * 8);
+  const size_t o_slot = c.take(slot_doubles(nx, ny, kSlotSkews) * 8);
+  char *ws = solve_scratch(ctx, c.at);
+  if (!ws) return 1;
+  std::vector<char> h(sizeof(SolveItem) + (nax + 3 * (size_t)nr) * 8);
+  SolveItem *hi = reinterpret_cast<SolveItem *>(h.data());
+  double *ax = reinterpret_cast<double *>(h.data() + sizeof(SolveItem)), *rec = ax + nax;
+  for (int i = 0; i < nx; ++i) ax[i] = xd[i] / 180.0 * kPiF;
+  for (int j = 0; j < ny; ++j) ax[nx + j] = yd[j] / 180.0 * kPiF;
+  std::memcpy(ax + nx + ny, xd, nx * 8);
+  std::memcpy(ax + 2 * nx + ny, yd, ny * 8);
+  if (nr) {
+    std::memcpy(rec, xr, nr * 8);
+    std::memcpy(rec + nr, yr, nr * 8);
+    std::memcpy(rec + 2 * (size_t)nr, rhs, nr * 8);
+  }
+  double *dax = reinterpret_cast<double *>(ws + o_item + sizeof(SolveItem)), *drec = dax + nax;
+  double *trig = reinterpret_cast<double *>(ws + o_trig);
+  double *in = reinterpret_cast<double *>(ws + o_in), *abc = reinterpret_cast<double *>(ws + o_abc);
+  double *slot = reinterpret_cast<double *>(ws + o_slot);
+  SlotDesc D{};
+  D.g = Grid{nx, ny, ax[1] - ax[0], ax[nx + 1] - ax[nx], dax, dax + nx, dax + nx + ny,
+             dax + 2 * nx + ny, trig, trig + ny};
+  D.sg = sg;
+  D.pskew = reinterpret_cast<double *>(ws + o_ps);
+  D.fun = in + 3 * N;
+  D.skew = slot;
+  double *nat = slot + (size_t)kSlotSkews * SE;
+  D.T = nat + kNatT * N;
+  D.Ta = nat + kNatTa * N;
+  D.Td = nat + kNatTd * N;
+  D.delta = nat + kNatDelta * N;
+  D.aux = nat + kSlotNat * N;
+  D.slot_skews = kSlotSkews;
+  D.aux_len = aux_len(nx, ny);
+  D.x0 = x0;
+  D.y0 = y0;
+  D.nr = nr;
+  D.recx = drec;
+  D.recy = drec + nr;
+  D.rhs_adj = drec + 2 * (size_t)nr;
+  S.status = reinterpret_cast<int *>(ws + o_item + offsetof(SolveItem, status));
+  D.status = S.status;
+  D.iters = S.status + 1;
+  hi->desc = D;
+  hi->status = SATT_OK;
+  std::memset(hi->iters, 0, sizeof hi->iters);
+  S.D = D;
+  S.desc = reinterpret_cast<SlotDesc *>(ws + o_item);
+  S.gd = GroupDims{1, SE, N, std::max(nx, ny), ny, sg.ns};
+  for (int st = 0; st < kStages; ++st) {
+    S.gd.waves[st] = team_waves(kMaxTeam, ny, sg.ns, st);
+    S.gd.depth[st] = kDeepPrefetch;
+  }
+  const hipStream_t s = ctx->stream;
+  HIPCHK(ctx, hipMemcpyAsync(ws + o_item, h.data(), h.size(), hipMemcpyHostToDevice, s));
+  const double *src[4] = {spha, sphb, sphc, fun};
+  for (int q = 0; q < (fun ? 4 : 3); ++q)
+    HIPCHK(ctx, hipMemcpyAsync(in + q * N, src[q], N * 8, hipMemcpyHostToDevice, s));
+  launch_grid_trig(s, D.g, trig, trig + ny);
+  launch_metric_fields(s, D.g, in, in + N, in + 2 * N, abc, abc + N, abc + 2 * N);
+  // an adjoint has no slowness, and its sweeps read none of the fields made of it
+  const PeriodFields pf{abc, abc + N, abc + 2 * N, fun ? in + 3 * N : abc, nullptr};
+  launch_period_skew(s, D.g, sg, 1, pf, reinterpret_cast<double *>(ws + o_ps), nullptr);
+  HIPCHK(ctx, hipGetLastError());
+  return SATT_OK;
+}
+
+// The solve's field, status and iteration count back on the host.
+int strip_solve_end(satt_ctx *ctx, const StripSolve &S, const double *field, double *out,
+                    int which, int &status, int &iters) {
+  int hs[7];
+  HIPCHK(ctx, hipMemcpyAsync(hs, S.status, sizeof hs, hipMemcpyDeviceToHost, ctx->stream));
+  HIPCHK(ctx, hipMemcpyAsync(out, field, (size_t)S.D.g.nx * S.D.g.ny * 8, hipMemcpyDeviceToHost,
+                             ctx->stream));
+  TRY(sync_status(ctx));
+  status = hs[0];
+  iters = hs[1 + which];
+  return SATT_OK;
+}
+
+// The same solves by the one-workgroup kernels.
+int plain_fwd(satt_ctx *ctx, const double *xx_deg, const double *yy_deg, int nx, int ny,
+              const double *spha, const double *sphb, const double *sphc, const double *fun,
+              double x0_deg, double y0_deg, double *T, int &status, int &iters) {
   const size_t N = (size_t)nx * ny;
   OneSolve o;
   TRY(make_grid(ctx, xx_deg, yy_deg, nx, ny, o.dg));
@@ -322,21 +477,15 @@ extern "C" int satt_fwd_lonlat(satt_ctx *ctx, const double *xx_deg, const double
   HIPCHK(ctx, hipMemcpyAsync(&hi, ibase, sizeof hi, hipMemcpyDeviceToHost, ctx->stream));
   HIPCHK(ctx, hipMemcpyAsync(T, fw.T, N * 8, hipMemcpyDeviceToHost, ctx->stream));
   TRY(sync_status(ctx));
-  if (iters) *iters = hi.it;
-  if (hi.st != SATT_OK) fail(ctx, hi.st, "satt_fwd_lonlat: %s", status_text(hi.st));
-  return hi.st;
+  status = hi.st;
+  iters = hi.it;
+  return SATT_OK;
 }
 
-extern "C" int satt_adj_lonlat(satt_ctx *ctx, const double *xx_deg, const double *yy_deg,
-                               int nx, int ny, const double *spha, const double *sphb,
-                               const double *sphc, const double *T, const double *xrec_deg,
-                               const double *yrec_deg, const double *src_adj, int nr,
-                               double *Ta, int *iters) {
-  if (!ctx) return SATT_E_ARG;
-  if (bad_fields(nx, ny, spha, sphb, sphc) || !T || !Ta || nr < 0 ||
-      (nr > 0 && (!xrec_deg || !yrec_deg || !src_adj)))
-    return fail(ctx, SATT_E_ARG, "satt_adj_lonlat: bad arguments");
-  HIPCHK(ctx, hipSetDevice(ctx->device));
+int plain_adj(satt_ctx *ctx, const double *xx_deg, const double *yy_deg, int nx, int ny,
+              const double *spha, const double *sphb, const double *sphc, const double *T,
+              const double *xrec_deg, const double *yrec_deg, const double *src_adj, int nr,
+              double *Ta, int &status, int &iters) {
   const size_t N = (size_t)nx * ny;
   OneSolve o;
   TRY(make_grid(ctx, xx_deg, yy_deg, nx, ny, o.dg));
@@ -371,9 +520,73 @@ extern "C" int satt_adj_lonlat(satt_ctx *ctx, const double *xx_deg, const double
   HIPCHK(ctx, hipMemcpyAsync(&hi, ibase, sizeof hi, hipMemcpyDeviceToHost, ctx->stream));
   HIPCHK(ctx, hipMemcpyAsync(Ta, aw.Ta, N * 8, hipMemcpyDeviceToHost, ctx->stream));
   TRY(sync_status(ctx));
-  if (iters) *iters = hi.it;
-  if (hi.st != SATT_OK) fail(ctx, hi.st, "satt_adj_lonlat: %s", status_text(hi.st));
-  return hi.st;
+  status = hi.st;
+  iters = hi.it;
+  return SATT_OK;
+}
+
+}  // namespace
+
+extern "C" int satt_fwd_lonlat(satt_ctx *ctx, const double *xx_deg, const double *yy_deg,
+                               int nx, int ny, const double *spha, const double *sphb,
+                               const double *sphc, const double *fun, double x0_deg,
+                               double y0_deg, double *T, int *iters) {
+  if (!ctx) return SATT_E_ARG;
+  if (bad_fields(nx, ny, spha, sphb, sphc) || !fun || !T)
+    return fail(ctx, SATT_E_ARG, "satt_fwd_lonlat: bad arguments");
+  HIPCHK(ctx, hipSetDevice(ctx->device));
+  int st = SATT_OK, it = 0, plain = ny > SATT_MAX_NY;
+  if (!plain) {
+    SolveScratchEnd end{ctx};
+    StripSolve S;
+    TRY(plain = strip_solve_setup(ctx, S, xx_deg, yy_deg, nx, ny, spha, sphb, sphc, fun, x0_deg,
+                                  y0_deg, 0, nullptr, nullptr, nullptr));
+    if (!plain) {
+      launch_fwd_setup(ctx->stream, S.desc, S.gd, false);
+      launch_fwd_strip(ctx->stream, S.desc, S.gd);
+      TRY(strip_solve_end(ctx, S, S.D.T, T, 0, st, it));
+    }
+  }
+  if (plain)
+    TRY(plain_fwd(ctx, xx_deg, yy_deg, nx, ny, spha, sphb, sphc, fun, x0_deg, y0_deg, T, st, it));
+  if (iters) *iters = it;
+  if (st != SATT_OK) fail(ctx, st, "satt_fwd_lonlat: %s", status_text(st));
+  return st;
+}
+
+extern "C" int satt_adj_lonlat(satt_ctx *ctx, const double *xx_deg, const double *yy_deg,
+                               int nx, int ny, const double *spha, const double *sphb,
+                               const double *sphc, const double *T, const double *xrec_deg,
+                               const double *yrec_deg, const double *src_adj, int nr,
+                               double *Ta, int *iters) {
+  if (!ctx) return SATT_E_ARG;
+  if (bad_fields(nx, ny, spha, sphb, sphc) || !T || !Ta || nr < 0 ||
+      (nr > 0 && (!xrec_deg || !yrec_deg || !src_adj)))
+    return fail(ctx, SATT_E_ARG, "satt_adj_lonlat: bad arguments");
+  HIPCHK(ctx, hipSetDevice(ctx->device));
+  int st = SATT_OK, it = 0, plain = ny > SATT_MAX_NY;
+  if (!plain) {
+    SolveScratchEnd end{ctx};
+    StripSolve S;
+    // a source at infinity: the output's mask takes no cell
+    const double far = HUGE_VAL;
+    TRY(plain = strip_solve_setup(ctx, S, xx_deg, yy_deg, nx, ny, spha, sphb, sphc, nullptr, far,
+                                  far, nr, xrec_deg, yrec_deg, src_adj));
+    if (!plain) {
+      HIPCHK(ctx, hipMemcpyAsync(S.D.T, T, (size_t)nx * ny * 8, hipMemcpyHostToDevice,
+                                 ctx->stream));
+      launch_time_skew(ctx->stream, S.desc, S.gd);
+      launch_adj_setup(ctx->stream, S.desc, S.gd, 0, false);
+      launch_adj_strip(ctx->stream, S.desc, S.gd, 0);
+      TRY(strip_solve_end(ctx, S, S.D.Ta, Ta, 1, st, it));
+    }
+  }
+  if (plain)
+    TRY(plain_adj(ctx, xx_deg, yy_deg, nx, ny, spha, sphb, sphc, T, xrec_deg, yrec_deg, src_adj,
+                  nr, Ta, st, it));
+  if (iters) *iters = it;
+  if (st != SATT_OK) fail(ctx, st, "satt_adj_lonlat: %s", status_text(st));
+  return st;
 }
 
 extern "C" int satt_mask(satt_ctx *ctx, const double *xx, const double *yy, int nx, int ny,

@@ -2100,11 +2100,30 @@ __global__ __launch_bounds__(256) void k_item_kernel(const SlotDesc *sd) {
   D.kern[k] = 0.0 + D.Ta[k] / (v * v);
 }
 
+// A slot's T from natural layout into one of its skews (blockIdx.y); padding
+// elements get zeros.
+__global__ __launch_bounds__(256) void k_time_skew(const SlotDesc *sd) {
+  const SlotDesc D = sd[blockIdx.z];
+  const SkewGeom &sg = D.sg;
+  const size_t SE = sg.skew_elems(), e = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  if (e >= SE) return;
+  const int sk = blockIdx.y, l = (int)(e & 63);
+  const int r = (int)((e >> 6) % sg.R), i = 64 * (int)((e >> 6) / sg.R) + l;
+  const int j = sk == 0 ? r - l : r + l - 63;
+  const bool in = i < D.g.nx && j >= 0 && j < D.g.ny;
+  gm(D.skew)[(sk == 0 ? kSkTP : kSkTM) * SE + e] = in ? gm(D.T)[i + (size_t)D.g.nx * j] : 0.0;
+}
+
 }  // namespace
 
 void launch_item_kernel(hipStream_t s, const SlotDesc *sd, const GroupDims &gd) {
   hipLaunchKernelGGL(k_item_kernel, dim3((unsigned)((gd.max_n + 255) / 256), gd.count), dim3(256),
                      0, s, sd);
+}
+
+void launch_time_skew(hipStream_t s, const SlotDesc *sd, const GroupDims &gd) {
+  hipLaunchKernelGGL(k_time_skew, dim3((unsigned)((gd.max_se + 255) / 256), 2, gd.count),
+                     dim3(256), 0, s, sd);
 }
 
 void launch_period_skew(hipStream_t s, const Grid &g, const SkewGeom &sg, int np,

@@ -5,6 +5,7 @@ a candidate is left out by the narrowest margins or may not be left out."""
 import numpy as np
 import pytest
 
+import oracle as O
 import satt
 import satt_workloads as W
 
@@ -57,6 +58,42 @@ def test_sweeps_equal_the_full_update(ctx, kind, nx, ny, d, lat, waves):
     if kind != "nan":
         np.testing.assert_array_equal(out[0]["adj_s"], out[1]["adj_s"])
     for k in range(4):
-        Tk, it, _ = ctx.fwd(xg, yg, m11, m22, -m12, 1.0 / v, b["item_srcx"][k], b["item_srcy"][k])
-        np.testing.assert_array_equal(T[0][k], Tk)
-        assert it == out[0]["iters"][k, 0]
+        solve = (xg, yg, m11, m22, -m12, 1.0 / v, b["item_srcx"][k], b["item_srcy"][k])
+        for entry in (ctx.fwd, ctx.fwd_noalloc):
+            Tk, it, _ = entry(*solve)
+            np.testing.assert_array_equal(T[0][k], Tk)
+            assert it == out[0]["iters"][k, 0]
+
+
+@pytest.mark.parametrize("nx,ny,nr", [(40, 33, 0), (65, 30, 1), (129, 3, 12), (3, 70, 5), (70, 41, 700)])
+def test_adjoint_entry_point_equals_the_sequential_sweeps(ctx, nx, ny, nr):
+    """satt_adj_lonlat, without receivers, with more of them than a workgroup's
+    entries hold, several to a cell, on grids of one interior row or column."""
+    rng = np.random.default_rng(nx + ny)
+    xg, yg = 100.0 + 0.02 * np.arange(nx), 10.0 + 0.02 * np.arange(ny)
+    one, zero = np.ones((nx, ny)), np.zeros((nx, ny))
+    # times from a point inside (a grid of three rows has no forward solution)
+    T = 37.0 * np.hypot(xg[:, None] - xg[nx // 2] - 0.003, yg[None] - yg[ny // 2] - 0.004)
+    T = np.asfortranarray(T * (1 + 0.01 * rng.uniform(size=(nx, ny))))
+    xr, yr = rng.uniform(xg[0], xg[-2], nr), rng.uniform(yg[0], yg[-2], nr)
+    sa = rng.standard_normal(nr)
+    a, b, c, delta = ctx.adj_setup_fields(xg, yg, one, one, zero, xr, yr, sa)
+    want, it_o, _ = O.adj_pre(xg, yg, a, b, c, T, delta)
+    got, it, _ = ctx.adj(xg, yg, one, one, zero, T, xr, yr, sa)
+    assert it == it_o
+    np.testing.assert_array_equal(got, want)
+
+
+def test_solves_past_the_batched_row_limit(ctx):
+    """More rows than the batched sweeps take: the one-workgroup kernels."""
+    nx, ny = 4, 10250
+    xg, yg = 100.0 + 0.002 * np.arange(nx), 0.002 * np.arange(ny)
+    one, zero = np.ones((nx, ny)), np.zeros((nx, ny))
+    sx, sy = xg[1] + 0.001, yg[5000] + 0.0007
+    T, it, _ = ctx.fwd(xg, yg, one, one, zero, one / 3.0, sx, sy)
+    To, it_o, _ = O.fwd(xg, yg, one, one, zero, one / 3.0, sx, sy)
+    assert it == it_o
+    assert np.max(np.abs(T - To)) <= 1e-9 * np.max(To)
+    Ta, _, _ = ctx.adj(xg, yg, one, one, zero, To, [xg[2]], [yg[100] + 0.001], [1.0])
+    Tao, _, _ = O.adj(xg, yg, one, one, zero, To, [xg[2]], [yg[100] + 0.001], [1.0])
+    assert np.max(np.abs(Ta - Tao)) <= 1e-8 * np.max(np.abs(Tao))
