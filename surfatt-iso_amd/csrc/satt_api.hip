@@ -297,14 +297,16 @@ bool bad_fields(int nx, int ny, const void *a, const void *b, const void *c) {
 
 namespace {
 
-// One forward or adjoint solve on the batched sweeps: a launch group of one
-// slot whose team takes every strip of the grid it can.  The same bits as
-// the one-workgroup kernels (k_forward, k_adjoint), which step a barrier per
-// anti-diagonal on natural-layout fields; MI355X, forward and adjoint call
-// after another: 41^2 4.3 -> 2.5 ms, 401 x 343 101 -> 34.6 ms (device: forward
-// 74 -> 24.4, adjoint 25.9 -> 8.7), bound by the latency of a team's steps.
-// Grids past SATT_MAX_NY rows, and those whose skewed fields do not fit the
-// device, take those kernels.
+// One forward or adjoint solve: a launch group of one slot.  Where a strip's
+// tau fits LDS and the strips a channel each (quad_fits: to 1024 x 1231) it
+// runs across compute units (satt_quad.hip), else, or where a wait there ended
+// at its limit, on the batched sweeps with a team that takes every strip of
+// the grid it can.  The same bits as the one-workgroup kernels (k_forward,
+// k_adjoint), which step a barrier per anti-diagonal on natural-layout fields.
+// MI355X, one call of each after another, those kernels / batched sweeps /
+// across units: 41^2 4.3 / 2.5 / 1.3 ms, 401 x 343 101 / 34.6 / 12.3 ms, bound
+// by the latency of a step.  Grids past SATT_MAX_NY rows, and those whose
+// skewed fields do not fit the device, take the one-workgroup kernels.
 constexpr size_t kSolveKeepBytes = (size_t)256 << 20;
 
 // Pieces of the per-solve scratch, each on a 256-byte boundary.
@@ -348,19 +350,21 @@ struct SolveItem {
   int status, iters[6];
 };
 
-// The solve's descriptor, axes and receivers (rec: 3*nr values, or null) on
-// the device, the metric and the period's skewed fields; status SATT_OK, an
-// error, or 1 where the scratch does not fit the device.
+// The solve's descriptor, axes and receivers on the device, and the metric;
+// status SATT_OK, an error, or 1 where the scratch does not fit the device.
 struct StripSolve {
   GroupDims gd{};
   SlotDesc D{}, *desc = nullptr;
+  PeriodFields pf{};
+  char *quad = nullptr;   // scratch of launch_fwd_quad, if asked for
+  double *pskew = nullptr;
   int *status = nullptr;  // and the item's iteration counts behind it
 };
 
 int strip_solve_setup(satt_ctx *ctx, StripSolve &S, const double *xd, const double *yd, int nx,
                       int ny, const double *spha, const double *sphb, const double *sphc,
                       const double *fun, double x0, double y0, int nr, const double *xr,
-                      const double *yr, const double *rhs) {
+                      const double *yr, const double *rhs, bool quad) {
   if (!xd || !yd) return fail(ctx, SATT_E_ARG, "bad grid axes");
   const size_t N = (size_t)nx * ny, nax = 2 * ((size_t)nx + ny);
   const SkewGeom sg = make_skew_geom(nx, ny);
@@ -370,6 +374,7 @@ int strip_solve_setup(satt_ctx *ctx, StripSolve &S, const double *xd, const doub
   const size_t o_trig = c.take(2 * (size_t)ny * 8), o_in = c.take(4 * N * 8);
   const size_t o_abc = c.take(3 * N * 8), o_ps = c.take(2 * (size_t)kPF * SE * 8);
   const size_t o_slot = c.take(slot_doubles(nx, ny, kSlotSkews) * 8);
+  const size_t o_quad = c.take(quad ? quad_scratch_bytes(nx, ny) : 0);
   char *ws = solve_scratch(ctx, c.at);
   if (!ws) return 1;
   std::vector<char> h(sizeof(SolveItem) + (nax + 3 * (size_t)nr) * 8);
@@ -430,10 +435,16 @@ int strip_solve_setup(satt_ctx *ctx, StripSolve &S, const double *xd, const doub
   launch_grid_trig(s, D.g, trig, trig + ny);
   launch_metric_fields(s, D.g, in, in + N, in + 2 * N, abc, abc + N, abc + 2 * N);
   // an adjoint has no slowness, and its sweeps read none of the fields made of it
-  const PeriodFields pf{abc, abc + N, abc + 2 * N, fun ? in + 3 * N : abc, nullptr};
-  launch_period_skew(s, D.g, sg, 1, pf, reinterpret_cast<double *>(ws + o_ps), nullptr);
+  S.pf = PeriodFields{abc, abc + N, abc + 2 * N, fun ? in + 3 * N : abc, nullptr};
+  S.pskew = reinterpret_cast<double *>(ws + o_ps);
+  S.quad = quad ? ws + o_quad : nullptr;
   HIPCHK(ctx, hipGetLastError());
   return SATT_OK;
+}
+
+// The period's skewed fields, for the strip kernels.
+void strip_solve_skew(satt_ctx *ctx, const StripSolve &S) {
+  launch_period_skew(ctx->stream, S.D.g, S.D.sg, 1, S.pf, S.pskew, nullptr);
 }
 
 // The solve's field, status and iteration count back on the host.
@@ -540,8 +551,14 @@ extern "C" int satt_fwd_lonlat(satt_ctx *ctx, const double *xx_deg, const double
     SolveScratchEnd end{ctx};
     StripSolve S;
     TRY(plain = strip_solve_setup(ctx, S, xx_deg, yy_deg, nx, ny, spha, sphb, sphc, fun, x0_deg,
-                                  y0_deg, 0, nullptr, nullptr, nullptr));
-    if (!plain) {
+                                  y0_deg, 0, nullptr, nullptr, nullptr, quad_fits(nx, ny)));
+    if (!plain && S.quad) {
+      launch_fwd_quad(ctx->stream, S.desc, S.gd, S.D, S.pf, S.quad);
+      TRY(strip_solve_end(ctx, S, S.D.T, T, 0, st, it));
+    }
+    if (!plain && (!S.quad || st == SATT_E_TEAM_WAIT)) {
+      launch_zero(ctx->stream, S.status, sizeof(int));
+      strip_solve_skew(ctx, S);
       launch_fwd_setup(ctx->stream, S.desc, S.gd, false);
       launch_fwd_strip(ctx->stream, S.desc, S.gd);
       TRY(strip_solve_end(ctx, S, S.D.T, T, 0, st, it));
@@ -571,10 +588,17 @@ extern "C" int satt_adj_lonlat(satt_ctx *ctx, const double *xx_deg, const double
     // a source at infinity: the output's mask takes no cell
     const double far = HUGE_VAL;
     TRY(plain = strip_solve_setup(ctx, S, xx_deg, yy_deg, nx, ny, spha, sphb, sphc, nullptr, far,
-                                  far, nr, xrec_deg, yrec_deg, src_adj));
-    if (!plain) {
+                                  far, nr, xrec_deg, yrec_deg, src_adj, quad_fits(nx, ny)));
+    if (!plain)
       HIPCHK(ctx, hipMemcpyAsync(S.D.T, T, (size_t)nx * ny * 8, hipMemcpyHostToDevice,
                                  ctx->stream));
+    if (!plain && S.quad) {
+      launch_adj_quad(ctx->stream, S.desc, S.gd, S.D, S.pf, S.quad);
+      TRY(strip_solve_end(ctx, S, S.D.Ta, Ta, 1, st, it));
+    }
+    if (!plain && (!S.quad || st == SATT_E_TEAM_WAIT)) {
+      launch_zero(ctx->stream, S.status, sizeof(int));
+      strip_solve_skew(ctx, S);
       launch_time_skew(ctx->stream, S.desc, S.gd);
       launch_adj_setup(ctx->stream, S.desc, S.gd, 0, false);
       launch_adj_strip(ctx->stream, S.desc, S.gd, 0);

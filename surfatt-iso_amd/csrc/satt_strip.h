@@ -90,11 +90,81 @@ int team_waves(int want, int ny, int ns, int stage);
 // plan's own inputs and leaves the plan set to them (satt_api.hip).
 int tune_plan_shapes(satt_plan *P, satt_tune_result &r);
 
+// T0, T0x, T0y of one cell (src/eikon_solver_2d.f90:845-857) from the
+// row's sin/cos of the latitude and the column's sin/cos of the longitude
+// difference: the expressions of t0_cell_s, with the same operand values.
+__device__ __forceinline__ void t0_cell_tab(double sy, double cy, double sdx, double cdx,
+                                            double sy0, double cy0, double fun0, double &T0,
+                                            double &T0x, double &T0y) {
+  const double t = sy * sy0 + cy * cy0 * cdx;
+  double tc = t < 1.0 ? t : 1.0;
+  tc = tc > -1.0 ? tc : -1.0;
+  T0 = acos(tc) * kREarth * fun0;
+  if (T0 == 0) {
+    T0x = 0;
+    T0y = 0;
+  } else {
+    const double s = sqrt(1 - t * t);
+    T0x = -(1.0 / s * cy * cy0 * (-1.0) * sdx * kREarth * fun0);
+    T0y = -(1.0 / s * (cy * sy0 - sy * cy0 * cdx) * kREarth * fun0);
+  }
+}
+
+// Face coefficients of one interior cell (src/eikon_solver_2d.f90:1348-1370)
+// from T at the 3x3 neighbourhood and the metric at the faces, and the sweep
+// denominator d = (a2p-a1m)/dx + (b2p-b1m)/dy (:1392), stored as 0 where
+// abs(d) < eps (:1394-1395).
+__device__ __forceinline__ void adj_coef_v(double Tk, double TW, double TE, double TS, double TN,
+                                           double TWS, double TWN, double TES, double TEN,
+                                           double ak, double aW, double aE, double bk, double bS,
+                                           double bN, double ck, double cW, double cE, double cS,
+                                           double cN, double dx, double dy, double *out) {
+  const double a1 = -((Tk - TW) / dx * (ak + aW) / 2) + (TN - TS + TWN - TWS) / (4 * dy) * (ck + cW) / 2;
+  const double a2 = -((TE - Tk) / dx * (aE + ak) / 2) + (TEN - TES + TN - TS) / (4 * dy) * (cE + ck) / 2;
+  const double b1 = -((Tk - TS) / dy * (bk + bS) / 2) + (TE - TW + TES - TWS) / (4 * dx) * (ck + cS) / 2;
+  const double b2 = -((TN - Tk) / dy * (bN + bk) / 2) + (TEN - TWN + TE - TW) / (4 * dx) * (cN + ck) / 2;
+  const double a1m = (a1 - fabs(a1)) / 2, a2p = (a2 + fabs(a2)) / 2;
+  const double b1m = (b1 - fabs(b1)) / 2, b2p = (b2 + fabs(b2)) / 2;
+  const double d = (a2p - a1m) / dx + (b2p - b1m) / dy;
+  out[0] = a1; out[1] = a2; out[2] = b1; out[3] = b2;
+  out[4] = fabs(d) < kAdjEps ? 0.0 : d;
+}
+
+__device__ __forceinline__ size_t skidx(int c, int r, int l, int R) {
+  return ((size_t)c * R + r) * 64 + l;
+}
+
+// Position of cell (i, j) in skew sk (0 plus, 1 minus).  For 64 lanes of one
+// strip and a common offset (di, dj) the positions of (i+di, j+dj) are one
+// contiguous run, except for the lane that crosses into the next strip.
+__device__ __forceinline__ size_t skpos(int sk, int i, int j, int R) {
+  const int c = i >> 6, l = i & 63;
+  const int r = sk == 0 ? j + l : j - l + 63;
+  return skidx(c, r, l, R);
+}
+
+// One FP64 solve across compute units (satt_quad.hip): the forward, four lanes
+// per cell, on the slot's tables and the natural-layout fields a, b, c, fun of
+// pf, and the adjoint on its natural T, its receivers and a, b, c.  T or Ta,
+// status and iteration count as launch_fwd_strip's and launch_adj_strip's, in
+// natural layout only and without the mask.  A status of kETeamWait (a wave of
+// the launch was not running) leaves the field unset.  D: the slot's
+// descriptor sd on the host.  For grids that quad_fits; scratch:
+// quad_scratch_bytes.
+constexpr int kQuadMaxStrips = 64;  // waves of a launch: a quarter of the CUs
+bool quad_fits(int nx, int ny);
+size_t quad_scratch_bytes(int nx, int ny);
+void launch_fwd_quad(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, const SlotDesc &D,
+                     const PeriodFields &pf, void *scratch);
+void launch_adj_quad(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, const SlotDesc &D,
+                     const PeriodFields &pf, void *scratch);
+
 // Batched kernels over the slots of a launch group (satt_strip.hip); all
 // asynchronous on `s`.  Forward: setup (per-item tables, then T0 skews and
 // the tau init, one thread per element), then the sweeps: k_fwd_strip
 // (FP64), or k_fwd_mixed32 (FP32 phase) followed by k_fwd_polish (FP64 to
 // the reference's stop rule).
+void launch_fwd_prep(hipStream_t s, const SlotDesc *sd, const GroupDims &gd);  // the tables only
 void launch_fwd_setup(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, bool mixed);
 void launch_fwd_strip(hipStream_t s, const SlotDesc *sd, const GroupDims &gd);
 void launch_fwd_mixed32(hipStream_t s, const SlotDesc *sd, const GroupDims &gd);
@@ -105,6 +175,8 @@ void launch_fwd_polish(hipStream_t s, const SlotDesc *sd, const GroupDims &gd);
 // natural layout and scattered into the coefficient fields), then the
 // sweeps: k_adj_strip (FP64), or k_adj_mixed32 followed by k_adj_polish
 // (one FP64 iteration).  Output Ta (which 0) or Td (which 1), masked.
+void launch_adj_source(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, int which,
+                       bool mixed);  // the delta source only
 void launch_adj_setup(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, int which,
                       bool mixed);
 void launch_adj_strip(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, int which);

@@ -145,10 +145,6 @@ __device__ __forceinline__ void wave_fence() {
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
 }
 
-__device__ __forceinline__ size_t skidx(int c, int r, int l, int R) {
-  return ((size_t)c * R + r) * 64 + l;
-}
-
 // The index unchanged, hidden from the optimizer: a load at a selected
 // index whose other choice is an index loaded anyway would otherwise become
 // that load plus a second one behind a branch.
@@ -458,15 +454,6 @@ __device__ __forceinline__ void t0_cell_s(double xxi, double yyj, double x0, dou
     T0x = -(1.0 / s * cy * cy0 * (-1.0) * sdx * kREarth * fun0);
     T0y = -(1.0 / s * (cy * sy0 - sy * cy0 * cdx) * kREarth * fun0);
   }
-}
-
-// Position of cell (i, j) in skew sk (0 plus, 1 minus).  For 64 lanes of one
-// strip and a common offset (di, dj) the positions of (i+di, j+dj) are one
-// contiguous run, except for the lane that crosses into the next strip.
-__device__ __forceinline__ size_t skpos(int sk, int i, int j, int R) {
-  const int c = i >> 6, l = i & 63;
-  const int r = sk == 0 ? j + l : j - l + 63;
-  return skidx(c, r, l, R);
 }
 
 // The waves of one workgroup working on one item (a team of W waves).  The
@@ -1102,26 +1089,6 @@ __global__ __launch_bounds__(64) void k_fwd_prep(const SlotDesc *sd) {
   }
 }
 
-// T0, T0x, T0y of one cell (src/eikon_solver_2d.f90:845-857) from the
-// row's sin/cos of the latitude and the column's sin/cos of the longitude
-// difference: the expressions of t0_cell_s, with the same operand values.
-__device__ __forceinline__ void t0_cell_tab(double sy, double cy, double sdx, double cdx,
-                                            double sy0, double cy0, double fun0, double &T0,
-                                            double &T0x, double &T0y) {
-  const double t = sy * sy0 + cy * cy0 * cdx;
-  double tc = t < 1.0 ? t : 1.0;
-  tc = tc > -1.0 ? tc : -1.0;
-  T0 = acos(tc) * kREarth * fun0;
-  if (T0 == 0) {
-    T0x = 0;
-    T0y = 0;
-  } else {
-    const double s = sqrt(1 - t * t);
-    T0x = -(1.0 / s * cy * cy0 * (-1.0) * sdx * kREarth * fun0);
-    T0y = -(1.0 / s * (cy * sy0 - sy * cy0 * cdx) * kREarth * fun0);
-  }
-}
-
 // Tiled per-element launches (the forward setup, the adjoint coefficient
 // build): a workgroup does a tile of kTileElems consecutive elements of one
 // skew of one slot (32 rows of a strip), so that the rows above and below a
@@ -1374,26 +1341,6 @@ __global__ __launch_bounds__(TEAM ? 64 * kMaxTeam : 64) void k_fwd_polish(const 
 }
 
 // ------------------------------------------------------------- adjoint
-
-// Face coefficients of one interior cell (src/eikon_solver_2d.f90:1348-1370)
-// from T at the 3x3 neighbourhood and the metric at the faces, and the sweep
-// denominator d = (a2p-a1m)/dx + (b2p-b1m)/dy (:1392), stored as 0 where
-// abs(d) < eps (:1394-1395).
-__device__ __forceinline__ void adj_coef_v(double Tk, double TW, double TE, double TS, double TN,
-                                           double TWS, double TWN, double TES, double TEN,
-                                           double ak, double aW, double aE, double bk, double bS,
-                                           double bN, double ck, double cW, double cE, double cS,
-                                           double cN, double dx, double dy, double *out) {
-  const double a1 = -((Tk - TW) / dx * (ak + aW) / 2) + (TN - TS + TWN - TWS) / (4 * dy) * (ck + cW) / 2;
-  const double a2 = -((TE - Tk) / dx * (aE + ak) / 2) + (TEN - TES + TN - TS) / (4 * dy) * (cE + ck) / 2;
-  const double b1 = -((Tk - TS) / dy * (bk + bS) / 2) + (TE - TW + TES - TWS) / (4 * dx) * (ck + cS) / 2;
-  const double b2 = -((TN - Tk) / dy * (bN + bk) / 2) + (TEN - TWN + TE - TW) / (4 * dx) * (cN + ck) / 2;
-  const double a1m = (a1 - fabs(a1)) / 2, a2p = (a2 + fabs(a2)) / 2;
-  const double b1m = (b1 - fabs(b1)) / 2, b2p = (b2 + fabs(b2)) / 2;
-  const double d = (a2p - a1m) / dx + (b2p - b1m) / dy;
-  out[0] = a1; out[1] = a2; out[2] = b1; out[3] = b2;
-  out[4] = fabs(d) < kAdjEps ? 0.0 : d;
-}
 
 // The mixed mode's update weights of one interior cell, for the form
 // Ta = k0 + kW*TaW + kE*TaE + kS*TaS + kN*TaN: the face coefficients of
@@ -2140,9 +2087,13 @@ void launch_grid_trig(hipStream_t s, const Grid &g, double *sy, double *cy) {
 namespace {
 }  // namespace
 
-void launch_fwd_setup(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, bool mixed) {
+void launch_fwd_prep(hipStream_t s, const SlotDesc *sd, const GroupDims &gd) {
   hipLaunchKernelGGL(k_fwd_prep, dim3((unsigned)((gd.max_nxy + 63) / 64), gd.count), dim3(64), 0,
                      s, sd);
+}
+
+void launch_fwd_setup(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, bool mixed) {
+  launch_fwd_prep(s, sd, gd);
   if (mixed)
     hipLaunchKernelGGL(k_fwd_setup<true>, tile_grid(gd), dim3(256), 0, s, sd, gd.count,
                        tiles_per_skew(gd));
@@ -2202,6 +2153,11 @@ void launch_fwd_polish(hipStream_t s, const SlotDesc *sd, const GroupDims &gd) {
   hipLaunchKernelGGL(k, dim3(gd.count), stage_block(gd, st), team_lds(gd, st, 8), s, sd);
 }
 
+void launch_adj_source(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, int which,
+                       bool mixed) {
+  hipLaunchKernelGGL(k_adj_source, dim3(gd.count), dim3(256), 0, s, sd, which, (int)mixed);
+}
+
 void launch_adj_setup(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, int which,
                       bool mixed) {
   if (mixed)
@@ -2210,7 +2166,7 @@ void launch_adj_setup(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, in
   else
     hipLaunchKernelGGL(k_adj_build, tile_grid(gd), dim3(256), 0, s, sd, gd.count,
                        tiles_per_skew(gd));
-  hipLaunchKernelGGL(k_adj_source, dim3(gd.count), dim3(256), 0, s, sd, which, (int)mixed);
+  launch_adj_source(s, sd, gd, which, mixed);
 }
 
 void launch_adj_strip(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, int which) {

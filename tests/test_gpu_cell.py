@@ -84,6 +84,33 @@ def test_adjoint_entry_point_equals_the_sequential_sweeps(ctx, nx, ny, nr):
     np.testing.assert_array_equal(got, want)
 
 
+@pytest.mark.parametrize("nx,ny", [
+    (3, 3), (15, 9), (16, 8), (17, 7), (32, 40), (33, 41), (4, 1231), (4, 1232), (1024, 5), (1025, 5)])
+def test_solve_across_compute_units_at_its_edges(ctx, nx, ny):
+    """satt_fwd_lonlat and satt_adj_lonlat on widths about a strip's 16 columns
+    and the largest sizes of that route and the first past it."""
+    rng = np.random.default_rng(nx + 7 * ny)
+    xg, yg = 100.0 + 0.01 * np.arange(nx), 5.0 + 0.01 * np.arange(ny)
+    one = np.ones((nx, ny))
+    v = rng.uniform(2.5, 4.5, (nx, ny))
+    c = rng.uniform(-0.3, 0.3, (nx, ny))
+    sx, sy = xg[(nx - 1) // 2] + 0.003, yg[(ny - 1) // 2] + 0.004
+    solve = (xg, yg, one, one, c, 1.0 / v, sx, sy)
+    T = 37.0 * np.hypot(xg[:, None] - sx, yg[None] - sy)
+    if min(nx, ny) > 3:
+        T, it, _ = ctx.fwd(*solve)
+        want, it_o, _ = ctx.fwd_noalloc(*solve)
+        assert it == it_o
+        np.testing.assert_array_equal(T, want)
+    xr, yr = rng.uniform(xg[0], xg[-2], 5), rng.uniform(yg[0], yg[-2], 5)
+    sa = rng.standard_normal(5)
+    ga, gb, gc, delta = ctx.adj_setup_fields(xg, yg, one, one, c, xr, yr, sa)
+    want, it_o, _ = O.adj_pre(xg, yg, ga, gb, gc, T, delta)
+    got, it, _ = ctx.adj(xg, yg, one, one, c, T, xr, yr, sa)
+    assert it == it_o
+    np.testing.assert_array_equal(got, want)
+
+
 def test_solves_past_the_batched_row_limit(ctx):
     """More rows than the batched sweeps take: the one-workgroup kernels."""
     nx, ny = 4, 10250
