@@ -307,7 +307,7 @@ __device__ __forceinline__ double fmav(double a, double b, double c) { return a 
 // update.  Operands are offsets dtau = tau - 1; zX, zY are the upwind
 // neighbours' T0.
 // The quotients and the root are satt_div.h's: a step's chain of them is half
-// as long as the compiler's, and gives the same bits.  MI355X, 401 x 343,
+// as long as the compiler's, and gives the same bits.  MI355X, 401^2,
 // FP32 phase of 800 solves 36.5 -> 33.4 ms, polish 14.9 -> 14.5.  To leave out
 // the quadrant, or its lesser root, where it cannot be accepted (as the FP64
 // cell does) took 33.2 ms: the waves wait for memory and each other by then.
@@ -484,6 +484,7 @@ struct Team {
   LMEM char *chan0;   // [W][ny] their T0 (forward; V)
   volatile LMEM int *cnt;   // [2][W] rows published by each wave in the sweep
   volatile LMEM int *stop;  // set when a wait ran out
+  volatile LMEM int *done;  // [W] sweeps each wave has ended, its strips copied
   LMEM double *part;        // [ns][3] per-strip residual terms
   __device__ bool multi() const { return W > 1; }
 };
@@ -493,7 +494,7 @@ constexpr int kTeamSpinLimit = 1 << 22;  // ~0.5 s of s_sleep per wait
 // LDS bytes of a team of W waves on grids up to ny rows and ns strips.
 __host__ __device__ inline size_t team_lds_bytes(int W, int ny, int ns, int vbytes) {
   if (W <= 1) return (size_t)2 * ny * vbytes;  // the two channels only
-  return (size_t)ns * 3 * 8 + (size_t)2 * W * ny * vbytes + (size_t)(2 * W + 2) * 4;
+  return (size_t)ns * 3 * 8 + (size_t)2 * W * ny * vbytes + (size_t)(3 * W + 2) * 4;
 }
 
 // TEAM false: the one-wave form, with W = 1 known at compile time so that
@@ -513,23 +514,51 @@ __device__ inline Team team_init(void *lds, int ny, int ns, int vbytes) {
   T.chan0 = b + (size_t)T.W * ny * vbytes;
   T.cnt = (volatile LMEM int *)(b + (size_t)2 * T.W * ny * vbytes);
   T.stop = T.cnt + 2 * T.W;
+  T.done = T.stop + 1;
   if (TEAM) {
     if (threadIdx.x < 2 * (unsigned)T.W) T.cnt[threadIdx.x] = 0;
+    if (threadIdx.x < (unsigned)T.W) T.done[threadIdx.x] = 0;
     if (threadIdx.x == 0) *T.stop = 0;
     __syncthreads();
   }
   return T;
 }
 
-// Start of a sweep: clear this wave's count of the other set (used by the
-// previous sweep, which every wave has finished, and by the next one, which
-// starts after the barrier that ends this one).
+// Start of a sweep: clear this wave's count of the other set, used by the
+// previous sweep, which the wave that reads it has finished, and by the next
+// one, which that wave starts once it has read this wave's rows of this one
+// (or after the barrier that ends it).
 __device__ inline void team_sweep_begin(Team &T) {
   if (T.multi() && (threadIdx.x & 63) == 0) T.cnt[((T.sweep + 1) & 1) * T.W + T.w] = 0;
 }
 __device__ inline void team_sweep_end(Team &T) {
   ++T.sweep;
   __syncthreads();
+}
+// End of the first sweep of a pair in one x direction, this wave's strips
+// copied into the other skew: the second may start on them as soon as the next
+// wave has ended the first and copied too.  By then that wave has read the
+// channel rows that this one overwrites, and its strips' columns, which this
+// one's read as their old downstream neighbours, are in place.  A team is thus
+// filled strip by strip once for two sweeps, and the copies of the first
+// strips run beside the sweep of the last: with 7 strips of 401 rows on 7
+// waves a pair takes about 1380 steps, where a barrier after each sweep made
+// it 1700 and the copy's time.  MI355X, 800 solves at 401^2:
+// FP32 forward 33.2 -> 30.2 ms, FP32 adjoint 27.4 -> 22.4; 600 FP64 ones:
+// forward 56.4 -> 51.9, adjoint 44.1 -> 40.2.
+__device__ inline void team_sweep_turn(Team &T) {
+  ++T.sweep;
+  wave_fence();
+  if (T.multi()) {
+    T.done[T.w] = T.sweep;
+    volatile LMEM int *d = T.done + (T.w + 1) % T.W;
+    int spins = 0;
+    while (*d < T.sweep && !*T.stop) {
+      __builtin_amdgcn_s_sleep(2);
+      if (++spins > kTeamSpinLimit) *T.stop = 1;
+    }
+    wave_fence();
+  }
 }
 
 // Whether a wait of the team ran out (never for W = 1, which has no LDS).
@@ -701,6 +730,8 @@ __device__ __forceinline__ float as_f(unsigned u) { return __builtin_bit_cast(fl
 // Rows per batch: 16 in FP32, 8 in FP64 (measured at 401^2 x 4000 items and
 // 41^2 x 1600: 32 rows cost the FP32 kernels an occupancy step on the small
 // grid and gained nothing on the large one).
+// A wave copies the strips that it ran in the sweep before, x ascending from
+// the plus skew (FROM 0), descending from the minus skew.
 #ifndef SATT_COPY_KU_F32
 #define SATT_COPY_KU_F32 16
 #endif
@@ -714,7 +745,8 @@ __device__ __forceinline__ void skew_copy(const Team &T, const GMEM V *__restric
   constexpr int kU = sizeof(V) == 4 ? SATT_COPY_KU_F32 : SATT_COPY_KU_F64;
   constexpr int kRow = 64 * (int)sizeof(V);  // bytes of one skew row
   const unsigned strip_bytes = (unsigned)R * kRow;
-  for (int c = T.w; c < ns; c += T.W) {
+  for (int k = T.w; k < ns; k += T.W) {
+    const int c = FROM == 0 ? k : ns - 1 - k;
     const bool col = 64 * c + lane < nx;
     // destination row r holds the lane's cell j = r - jof, which sits in
     // source row j + sof
@@ -746,7 +778,6 @@ __device__ __forceinline__ void skew_copy(const Team &T, const GMEM V *__restric
       }
     }
   }
-  __syncthreads();
 }
 
 // Skew row of step t (uniform across lanes), see the layout note above.
@@ -1014,7 +1045,8 @@ __device__ __forceinline__ void fwd_strip_pass(const FwdCtx<V> &C, const Team &T
   wave_fence();
 }
 
-template <typename V, int XD, int YD, int MODE, bool UP, int PD>
+// TURN: the first sweep of a pair, which team_sweep_turn ends.
+template <typename V, int XD, int YD, int MODE, bool UP, int PD, bool TURN>
 __device__ __forceinline__ void fwd_sweep(const FwdCtx<V> &C, Team &T, GMEM V *tau, StripAcc &acc) {
   team_sweep_begin(T);
   for (int k = T.w; k < T.ns; k += T.W) {
@@ -1022,7 +1054,7 @@ __device__ __forceinline__ void fwd_sweep(const FwdCtx<V> &C, Team &T, GMEM V *t
     fwd_strip_pass<V, XD, YD, MODE, UP, PD>(C, T, k, tau, ss, sm);
     if (MODE == 2) team_strip_term(T, k, ss, sm, 0.0, acc);
   }
-  team_sweep_end(T);
+  if (!TURN) team_sweep_end(T);
 }
 
 // One iteration of four sweeps, (x+,y+), (x+,y-), (x-,y+), (x-,y-)
@@ -1035,14 +1067,16 @@ __device__ __forceinline__ bool fwd_iteration(const FwdCtx<V> &C, Team &T, GMEM 
                               bool first = false) {
   StripAcc acc;
   if (!UP && first)
-    fwd_sweep<V, 1, 1, UP ? 1 : 3, UP, PD>(C, T, tP, acc);
+    fwd_sweep<V, 1, 1, UP ? 1 : 3, UP, PD, true>(C, T, tP, acc);
   else
-    fwd_sweep<V, 1, 1, 1, UP, PD>(C, T, tP, acc);
+    fwd_sweep<V, 1, 1, 1, UP, PD, true>(C, T, tP, acc);
   skew_copy<V, 0>(T, tP, tM, C.nx, C.ny, C.R, T.ns, C.lane);
-  fwd_sweep<V, 1, -1, 0, UP, PD>(C, T, tM, acc);
-  fwd_sweep<V, -1, 1, 0, UP, PD>(C, T, tM, acc);
+  team_sweep_turn(T);
+  fwd_sweep<V, 1, -1, 0, UP, PD, false>(C, T, tM, acc);
+  fwd_sweep<V, -1, 1, 0, UP, PD, true>(C, T, tM, acc);
   skew_copy<V, 1>(T, tM, tP, C.nx, C.ny, C.R, T.ns, C.lane);
-  fwd_sweep<V, -1, -1, 2, UP, PD>(C, T, tP, acc);
+  team_sweep_turn(T);
+  fwd_sweep<V, -1, -1, 2, UP, PD, false>(C, T, tP, acc);
   const StripAcc r = team_strip_total(T, acc);
   const double l1 = r.s / (double)C.nx / (double)C.ny;
   // the FP32 phase stops at kMixFwdTolScale times the reference's tolerance:
@@ -1882,7 +1916,7 @@ __device__ void adj_strip_pass(const AdjCtx<V, CS> &C, const Team &T, int k, GME
   wave_fence();
 }
 
-template <typename V, int XD, int YD, int MODE, int PD, typename CS = V>
+template <typename V, int XD, int YD, int MODE, int PD, bool TURN, typename CS = V>
 __device__ void adj_sweep(const AdjCtx<V, CS> &C, Team &T, GMEM V *ta, StripAcc &acc) {
   team_sweep_begin(T);
   for (int k = T.w; k < T.ns; k += T.W) {
@@ -1890,7 +1924,7 @@ __device__ void adj_sweep(const AdjCtx<V, CS> &C, Team &T, GMEM V *ta, StripAcc 
     adj_strip_pass<V, XD, YD, MODE, PD, CS>(C, T, k, ta, ss, sm, sa);
     if (MODE == 2) team_strip_term(T, k, ss, sm, sa, acc);
   }
-  team_sweep_end(T);
+  if (!TURN) team_sweep_end(T);
 }
 
 // One iteration: (xdirec, ydirec) = (-1,-1), (-1,1), (1,-1), (1,1), x
@@ -1900,12 +1934,14 @@ template <typename V, bool SNAP, int PD, typename CS = V>
 __device__ void adj_iteration(const AdjCtx<V, CS> &C, Team &T, GMEM V *tP, GMEM V *tM, double &s,
                               double &m, double &a) {
   StripAcc acc;
-  adj_sweep<V, 1, 1, SNAP ? 1 : 0, PD, CS>(C, T, tP, acc);
+  adj_sweep<V, 1, 1, SNAP ? 1 : 0, PD, true, CS>(C, T, tP, acc);
   skew_copy<V, 0>(T, tP, tM, C.nx, C.ny, C.R, T.ns, C.lane);
-  adj_sweep<V, 1, -1, 0, PD, CS>(C, T, tM, acc);
-  adj_sweep<V, -1, 1, 0, PD, CS>(C, T, tM, acc);
+  team_sweep_turn(T);
+  adj_sweep<V, 1, -1, 0, PD, false, CS>(C, T, tM, acc);
+  adj_sweep<V, -1, 1, 0, PD, true, CS>(C, T, tM, acc);
   skew_copy<V, 1>(T, tM, tP, C.nx, C.ny, C.R, T.ns, C.lane);
-  adj_sweep<V, -1, -1, SNAP ? 2 : 0, PD, CS>(C, T, tP, acc);
+  team_sweep_turn(T);
+  adj_sweep<V, -1, -1, SNAP ? 2 : 0, PD, false, CS>(C, T, tP, acc);
   const StripAcc r = team_strip_total(T, acc);
   s = r.s;
   m = r.m;

@@ -41,6 +41,23 @@ def test_team_equals_one_wave(ctx, prec, nx, ny, dim):
         assert rel_l2(ref["adj_s"], o["adj_s"]) < 1e-8
 
 
+@pytest.mark.parametrize("prec", [satt.PREC_FP64, satt.PREC_MIXED])
+@pytest.mark.parametrize("nx,ny", [(65, 5), (320, 6), (449, 9), (129, 160)])
+def test_second_sweep_of_a_pair_started_early(ctx, prec, nx, ny):
+    """A wave starts the second sweep of a pair while later waves still run the
+    first: fewer rows than a strip has columns, as many waves as strips, fewer
+    (a wave with strips of both ends) and a strip of one column."""
+    b = shaped_batch(nx, ny, 3, 2, seed=nx + ny)
+    with ctx.plan(b, prec) as p:
+        p.run(True, True)
+        ref = p.results()
+        for W in (2, 3, (nx + 63) // 64):
+            p.set_waves(W)
+            for _ in range(2):
+                p.run(True, True)
+                same(p.results(), ref, 2, W)
+
+
 def test_team_multi_grid_and_graph(ctx):
     bs = parts(2)
     with ctx.plan_multi(bs, satt.PREC_MIXED) as p:
