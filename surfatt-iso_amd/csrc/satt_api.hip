@@ -304,7 +304,7 @@ namespace {
 // the grid it can.  The same bits as the one-workgroup kernels (k_forward,
 // k_adjoint), which step a barrier per anti-diagonal on natural-layout fields.
 // MI355X, one call of each after another, those kernels / batched sweeps /
-// across units: 41^2 4.3 / 2.5 / 1.3 ms, 401 x 343 101 / 34.6 / 12.3 ms, bound
+// across units: 41^2 4.3 / 2.5 / 1.2 ms, 401 x 343 101 / 34.6 / 11.2 ms, bound
 // by the latency of a step.  Grids past SATT_MAX_NY rows, and those whose
 // skewed fields do not fit the device, take the one-workgroup kernels.
 constexpr size_t kSolveKeepBytes = (size_t)256 << 20;
