@@ -78,6 +78,7 @@ struct satt_ctx {
   // kSolveKeepBytes and given back with the context
   void *solve_ws = nullptr;
   size_t solve_ws_bytes = 0;
+  int quit_strip = -1;            // satt_solve_fail_waits
 };
 
 bool satt::ctx_tune_lookup(satt_ctx *ctx, const TuneKey &k, TuneWaves &out) {
@@ -538,6 +539,12 @@ int plain_adj(satt_ctx *ctx, const double *xx_deg, const double *yy_deg, int nx,
 
 }  // namespace
 
+extern "C" int satt_solve_fail_waits(satt_ctx *ctx, int strip) {
+  if (!ctx) return SATT_E_ARG;
+  ctx->quit_strip = strip;
+  return SATT_OK;
+}
+
 extern "C" int satt_fwd_lonlat(satt_ctx *ctx, const double *xx_deg, const double *yy_deg,
                                int nx, int ny, const double *spha, const double *sphb,
                                const double *sphc, const double *fun, double x0_deg,
@@ -553,7 +560,7 @@ extern "C" int satt_fwd_lonlat(satt_ctx *ctx, const double *xx_deg, const double
     TRY(plain = strip_solve_setup(ctx, S, xx_deg, yy_deg, nx, ny, spha, sphb, sphc, fun, x0_deg,
                                   y0_deg, 0, nullptr, nullptr, nullptr, quad_fits(nx, ny)));
     if (!plain && S.quad) {
-      launch_fwd_quad(ctx->stream, S.desc, S.gd, S.D, S.pf, S.quad);
+      launch_fwd_quad(ctx->stream, S.desc, S.gd, S.D, S.pf, S.quad, ctx->quit_strip);
       TRY(strip_solve_end(ctx, S, S.D.T, T, 0, st, it));
     }
     if (!plain && (!S.quad || st == SATT_E_TEAM_WAIT)) {
@@ -593,7 +600,7 @@ extern "C" int satt_adj_lonlat(satt_ctx *ctx, const double *xx_deg, const double
       HIPCHK(ctx, hipMemcpyAsync(S.D.T, T, (size_t)nx * ny * 8, hipMemcpyHostToDevice,
                                  ctx->stream));
     if (!plain && S.quad) {
-      launch_adj_quad(ctx->stream, S.desc, S.gd, S.D, S.pf, S.quad);
+      launch_adj_quad(ctx->stream, S.desc, S.gd, S.D, S.pf, S.quad, ctx->quit_strip);
       TRY(strip_solve_end(ctx, S, S.D.Ta, Ta, 1, st, it));
     }
     if (!plain && (!S.quad || st == SATT_E_TEAM_WAIT)) {

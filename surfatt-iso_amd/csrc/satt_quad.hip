@@ -32,7 +32,9 @@
 // Every wait is for a wave of the same launch; all of them are resident
 // together, as a launch has at most kQuadMaxStrips one-wave workgroups, unless
 // other work holds the device.  A wait is bounded: past the bound the solve
-// ends with kETeamWait, and the caller takes the strip kernel.
+// ends with kETeamWait, and the caller takes the strip kernel.  Any strip may
+// be the one that gives up, in the wait for the last totals too, which the
+// others may find complete: so each gives the status its own part.
 #include "satt_div.h"
 #include "satt_internal.h"
 #include "satt_strip.h"
@@ -62,6 +64,7 @@ struct Quad {
   u64 *chan;      // [parity][strip][side][row][2]
   u64 *conv;      // [parity][strip][4]: the iteration's sum and maximum
   int *stop;      // a wait ran out
+  int quit;       // a strip that ends as if its last wait had run out, or -1
   double dx, dy;
 };
 
@@ -467,6 +470,7 @@ __global__ __launch_bounds__(64, 1) void k_quad(const SlotDesc *sd, Quad Q) {
     }
   }
   if (!conv) iter = kMaxIter;
+  if (S.k == Q.quit) ok = false;
   __syncthreads();
   if (ok)
     for (int e = S.lane; e < ny * kCols; e += 64) {
@@ -475,9 +479,14 @@ __global__ __launch_bounds__(64, 1) void k_quad(const SlotDesc *sd, Quad Q) {
       const double v = S.tau[e + kPadRows * kCols];
       if (i < nx) (ADJ ? D.Ta : D.T)[n] = ADJ ? v : v * Q.t0[n];
     }
-  if (S.k == 0 && S.lane == 0) {
-    *D.status = !ok ? kETeamWait : conv ? kOk : kWMaxIter;
-    D.iters[ADJ ? 1 : 0] = iter;
+  // kOk as uploaded, else the least of what the strips say: one that gave up
+  // has left its columns unwritten, whatever strip 0 found
+  if (S.lane == 0) {
+    if (!ok)
+      atomicMin(D.status, kETeamWait);
+    else if (S.k == 0 && !conv)
+      atomicCAS(D.status, kOk, kWMaxIter);
+    if (S.k == 0) D.iters[ADJ ? 1 : 0] = iter;
   }
 }
 
@@ -514,7 +523,7 @@ struct QuadLayout {
 size_t quad_scratch_bytes(int nx, int ny) { return QuadLayout(nx, ny).total; }
 
 namespace {
-Quad quad_of(const SlotDesc &D, void *scratch) {
+Quad quad_of(const SlotDesc &D, void *scratch, int quit) {
   const QuadLayout L(D.g.nx, D.g.ny);
   char *b = static_cast<char *>(scratch);
   Quad Q;
@@ -527,6 +536,7 @@ Quad quad_of(const SlotDesc &D, void *scratch) {
   Q.chan = reinterpret_cast<u64 *>(b + L.chan);
   Q.conv = reinterpret_cast<u64 *>(b + L.conv);
   Q.stop = reinterpret_cast<int *>(b + L.stop);
+  Q.quit = quit;
   Q.dx = D.g.dx;
   Q.dy = D.g.dy;
   return Q;
@@ -540,8 +550,8 @@ void quad_clear(hipStream_t s, const Quad &Q) {
 }  // namespace
 
 void launch_fwd_quad(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, const SlotDesc &D,
-                     const PeriodFields &pf, void *scratch) {
-  const Quad Q = quad_of(D, scratch);
+                     const PeriodFields &pf, void *scratch, int quit) {
+  const Quad Q = quad_of(D, scratch, quit);
   const size_t lanes = (size_t)Q.ns * Q.ny * 64;
   launch_fwd_prep(s, sd, gd);
   quad_clear(s, Q);
@@ -552,8 +562,8 @@ void launch_fwd_quad(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, con
 }
 
 void launch_adj_quad(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, const SlotDesc &D,
-                     const PeriodFields &pf, void *scratch) {
-  const Quad Q = quad_of(D, scratch);
+                     const PeriodFields &pf, void *scratch, int quit) {
+  const Quad Q = quad_of(D, scratch, quit);
   const size_t SE = D.sg.skew_elems(), cells = (size_t)Q.ns * Q.ny * kCols;
   launch_zero(s, D.skew + 5 * SE, SE * 8);
   launch_adj_source(s, sd, gd, 0, false);

@@ -150,14 +150,15 @@ __device__ __forceinline__ size_t skpos(int sk, int i, int j, int R) {
 // natural layout only and without the mask.  A status of kETeamWait (a wave of
 // the launch was not running) leaves the field unset.  D: the slot's
 // descriptor sd on the host.  For grids that quad_fits; scratch:
-// quad_scratch_bytes.
+// quad_scratch_bytes.  The slot's status is kOk before the launch.  quit: a
+// strip that gives up at its end (for tests), or -1.
 constexpr int kQuadMaxStrips = 64;  // waves of a launch: a quarter of the CUs
 bool quad_fits(int nx, int ny);
 size_t quad_scratch_bytes(int nx, int ny);
 void launch_fwd_quad(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, const SlotDesc &D,
-                     const PeriodFields &pf, void *scratch);
+                     const PeriodFields &pf, void *scratch, int quit);
 void launch_adj_quad(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, const SlotDesc &D,
-                     const PeriodFields &pf, void *scratch);
+                     const PeriodFields &pf, void *scratch, int quit);
 
 // Batched kernels over the slots of a launch group (satt_strip.hip); all
 // asynchronous on `s`.  Forward: setup (per-item tables, then T0 skews and

@@ -111,6 +111,43 @@ def test_solve_across_compute_units_at_its_edges(ctx, nx, ny):
     np.testing.assert_array_equal(got, want)
 
 
+def solve_pair(nx, ny, seed):
+    """(arguments of Context.fwd, of Context.adj after its T)"""
+    rng = np.random.default_rng(seed)
+    xg, yg = 100.0 + 0.01 * np.arange(nx), 5.0 + 0.01 * np.arange(ny)
+    one, c = np.ones((nx, ny)), rng.uniform(-0.3, 0.3, (nx, ny))
+    fun = 1.0 / rng.uniform(2.5, 4.5, (nx, ny))
+    xr, yr = rng.uniform(xg[0], xg[-2], 7), rng.uniform(yg[0], yg[-2], 7)
+    return ((xg, yg, one, one, c, fun, xg[nx // 2] + 0.003, yg[ny // 2] + 0.004),
+            (xr, yr, rng.standard_normal(7)))
+
+
+def recovered(nx, ny, **fail):
+    """Forward and adjoint with waits that run out, in a context whose scratch
+    holds another solve: what a call without such waits gives."""
+    solve, rec = solve_pair(nx, ny, nx)
+    with satt.Context(0) as c:
+        T, it, st = c.fwd(*solve)
+        Ta, ita, sta = c.adj(*solve[:5], T, *rec)
+        other, orec = solve_pair(nx, ny, nx + 1)
+        c.adj(*other[:5], c.fwd(*other)[0], *orec)
+        c.solve_fail_waits(**fail)
+        for _ in range(2):
+            got, it2, st2 = c.fwd(*solve)
+            assert (it2, st2) == (it, st)
+            np.testing.assert_array_equal(got, T)
+            got, it2, st2 = c.adj(*solve[:5], T, *rec)
+            assert (it2, st2) == (ita, sta)
+            np.testing.assert_array_equal(got, Ta)
+
+
+@pytest.mark.parametrize("nx,ny,strip", [(12, 9, 0), (70, 41, 0), (70, 41, 2), (70, 41, 4)])
+def test_a_strip_that_gives_up_is_not_lost(ctx, nx, ny, strip):
+    """The strip's columns are not written: the solve is done again on the
+    batched sweeps, also where the other strips ended in order."""
+    recovered(nx, ny, strip=strip)
+
+
 def test_solves_past_the_batched_row_limit(ctx):
     """More rows than the batched sweeps take: the one-workgroup kernels."""
     nx, ny = 4, 10250
