@@ -127,9 +127,10 @@ int satt_adj_lonlat(satt_ctx *ctx, const double *xx_deg, const double *yy_deg,
 
 /* For tests of the recovery: in the next satt_fwd_lonlat and satt_adj_lonlat
  * calls of this context, strip `strip` (16 columns of the grid) of a solve
- * across compute units ends as if its last wait for the others had run out;
- * -1, the default, none.  The results do not change. */
-int satt_solve_fail_waits(satt_ctx *ctx, int strip);
+ * across compute units ends as if its last wait for the others had run out
+ * (-1, the default: none), and with team != 0 a solve on the batched sweeps
+ * counts as one whose waits did.  The results do not change. */
+int satt_solve_fail_waits(satt_ctx *ctx, int strip, int team);
 
 /* satt_fwd_lonlat without any device allocation: the same kernels on the same
  * operands, hence the same T bit for bit.  No counterpart in the reference;

@@ -79,6 +79,7 @@ struct satt_ctx {
   void *solve_ws = nullptr;
   size_t solve_ws_bytes = 0;
   int quit_strip = -1;            // satt_solve_fail_waits
+  bool quit_team = false;
 };
 
 bool satt::ctx_tune_lookup(satt_ctx *ctx, const TuneKey &k, TuneWaves &out) {
@@ -307,7 +308,8 @@ namespace {
 // MI355X, one call of each after another, those kernels / batched sweeps /
 // across units: 41^2 4.3 / 2.5 / 1.2 ms, 401 x 343 101 / 34.6 / 11.2 ms, bound
 // by the latency of a step.  Grids past SATT_MAX_NY rows, and those whose
-// skewed fields do not fit the device, take the one-workgroup kernels.
+// skewed fields do not fit the device, take the one-workgroup kernels, and so
+// does a solve whose waits ran out in both of the others.
 constexpr size_t kSolveKeepBytes = (size_t)256 << 20;
 
 // Pieces of the per-solve scratch, each on a 256-byte boundary.
@@ -539,9 +541,10 @@ int plain_adj(satt_ctx *ctx, const double *xx_deg, const double *yy_deg, int nx,
 
 }  // namespace
 
-extern "C" int satt_solve_fail_waits(satt_ctx *ctx, int strip) {
+extern "C" int satt_solve_fail_waits(satt_ctx *ctx, int strip, int team) {
   if (!ctx) return SATT_E_ARG;
   ctx->quit_strip = strip;
+  ctx->quit_team = team != 0;
   return SATT_OK;
 }
 
@@ -569,6 +572,7 @@ extern "C" int satt_fwd_lonlat(satt_ctx *ctx, const double *xx_deg, const double
       launch_fwd_setup(ctx->stream, S.desc, S.gd, false);
       launch_fwd_strip(ctx->stream, S.desc, S.gd);
       TRY(strip_solve_end(ctx, S, S.D.T, T, 0, st, it));
+      plain = st == SATT_E_TEAM_WAIT || ctx->quit_team;
     }
   }
   if (plain)
@@ -610,6 +614,7 @@ extern "C" int satt_adj_lonlat(satt_ctx *ctx, const double *xx_deg, const double
       launch_adj_setup(ctx->stream, S.desc, S.gd, 0, false);
       launch_adj_strip(ctx->stream, S.desc, S.gd, 0);
       TRY(strip_solve_end(ctx, S, S.D.Ta, Ta, 1, st, it));
+      plain = st == SATT_E_TEAM_WAIT || ctx->quit_team;
     }
   }
   if (plain)

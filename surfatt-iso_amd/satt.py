@@ -188,9 +188,9 @@ class Context:
         self._check(st)
         return T, it.value, st
 
-    def solve_fail_waits(self, strip=-1):
-        """satt_solve_fail_waits: fwd and adj recover from a wait that ran out."""
-        self._check(self.lib.satt_solve_fail_waits(self.ptr, int(strip)))
+    def solve_fail_waits(self, strip=-1, team=False):
+        """satt_solve_fail_waits: fwd and adj recover from waits that ran out."""
+        self._check(self.lib.satt_solve_fail_waits(self.ptr, int(strip), int(team)))
 
     def fwd_noalloc(self, xx, yy, spha, sphb, sphc, fun, x0, y0):
         """satt_fwd_lonlat_noalloc (no device allocation) -> (T, iters, status)."""

@@ -148,6 +148,13 @@ def test_a_strip_that_gives_up_is_not_lost(ctx, nx, ny, strip):
     recovered(nx, ny, strip=strip)
 
 
+@pytest.mark.parametrize("nx,ny,strip", [(70, 41, 1), (1025, 5, -1)])
+def test_solves_whose_teams_give_up_too(ctx, nx, ny, strip):
+    """The one-workgroup kernels, which wait for nothing, are the last resort,
+    with and without a solve across compute units before."""
+    recovered(nx, ny, strip=strip, team=True)
+
+
 def test_solves_past_the_batched_row_limit(ctx):
     """More rows than the batched sweeps take: the one-workgroup kernels."""
     nx, ny = 4, 10250
