@@ -184,10 +184,15 @@ __device__ __forceinline__ double own_reg(double x) {
 //    which at the lesser root is -sqrt(delta)/2: where px and py have their
 //    neighbours' signs, chx and chy cannot both have them there.  And the
 //    greater root cannot lie below tau where 2 ea tau + eb < sqrt(delta).
-//    Both need ea > 0 and delta above 1e-12 eb^2: a root of delta is then
-//    1e-6 |eb| or more, against rounding of about 1e-15 |eb| in these
-//    terms; the second has a margin of 1e-6 beside.  A comparison with NaN
-//    is false, and the roots are evaluated.
+//    Both need ea > 0 and delta above 1e-12 (eb^2 + ea ff): a root of delta is
+//    then 7e-7 (|eb| + sqrt(ea ff)) or more.  eb and the tested components are
+//    sums whose terms may cancel; with p and q the vectors (px, py), (qx, qy)
+//    in the metric, (p.q)^2 + det (px qy - py qx)^2 = |p|^2 |q|^2, p.q = eb/2,
+//    and the second term is at most ea ff where delta >= 0, so that the terms
+//    are at most the metric's condition number times |eb| + sqrt(ea ff), and
+//    their rounding, about 1e-15 of them, stays below the root for condition
+//    numbers to 1e8.  The second has a margin of 1e-6 beside.  A comparison
+//    with NaN is false, and the roots are evaluated.
 //  - The greater one-sided value where it exceeds tau, and the lesser where
 //    its time falls short of the neighbour's, by more than 1e-12 of them.
 // One cell took 18 divisions and 4 square roots, 2100 cycles of a SIMD; in
@@ -242,7 +247,8 @@ __device__ __forceinline__ double fwd_cell_r(int i, int j, int nx, int ny, const
     const double delta = ebb - 4 * ea * ec;
     const double ea2 = 2 * ea;
     const bool one = ea > 0 && (sx[x] > 0 ? px[x] > 0 : px[x] < 0) &&
-                     (sy[y] > 0 ? py[y] > 0 : py[y] < 0) && delta > 1e-12 * ebb;
+                     (sy[y] > 0 ? py[y] > 0 : py[y] < 0) &&
+                     delta > 1e-12 * __builtin_fma(ea, ff, ebb);
     const double h = __builtin_fma(ea2, tnew, eb);
     const bool above = h < 0 || h * h < (1 - 1e-6) * delta;  // the greater root is above tau
     if (hx[x] && hy[y] && delta >= 0 && !(one && above)) {

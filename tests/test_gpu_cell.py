@@ -22,6 +22,10 @@ def model(kind, nx, ny, rng):
     if kind == "sheared":       # m12^2 within 2% of m11 m22, of either sign
         a, b = rng.uniform(0.5, 1, (nx, ny)), rng.uniform(0.5, 1, (nx, ny))
         return rng.uniform(2, 4, (nx, ny)), a, 0.99 * np.sqrt(a * b) * np.sign(rng.uniform(-1, 1, (nx, ny))), b
+    if kind == "oblique":       # condition numbers to 1e7, the long axis across the cells' diagonals
+        a, b = rng.uniform(0.5, 1, (nx, ny)), rng.uniform(0.5, 1, (nx, ny))
+        eps = 10.0 ** rng.uniform(-6.5, -2, (nx, ny))
+        return rng.uniform(2, 4, (nx, ny)), a, (1 - eps) * np.sqrt(a * b), b
     if kind == "indefinite":    # no metric at all: ea of either sign in some cells
         return rng.uniform(2, 4, (nx, ny)), one, np.where(rng.uniform(size=(nx, ny)) < 0.1, 1.2, 0.1), one
     if kind == "nan":
@@ -35,6 +39,7 @@ def model(kind, nx, ny, rng):
     ("ties", 41, 37, 0.05, 20.0), ("ties", 130, 20, 0.01, -1.0), ("smooth", 65, 64, 0.02, 60.0),
     ("smooth", 5, 70, 0.1, 0.0), ("smooth", 129, 6, 0.01, 10.0), ("rough", 64, 40, 0.01, 30.0),
     ("rough", 90, 35, 0.5, 40.0), ("sheared", 50, 66, 0.02, 20.0), ("sheared", 67, 31, 0.02, 20.0),
+    ("oblique", 48, 45, 0.02, 0.0), ("oblique", 70, 35, 0.02, 50.0),
     ("indefinite", 40, 33, 0.02, 20.0), ("nan", 33, 40, 0.02, 20.0),
 ])
 @pytest.mark.parametrize("waves", [1, 3])
