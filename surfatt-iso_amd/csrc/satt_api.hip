@@ -735,7 +735,7 @@ int geo_timer_read(satt_ctx *ctx, GeoTimer &t) {
 // evaluated on the host), the natural-layout output.
 struct GeoSmoothBufs {
   DBuf axes, tab, out;
-  int nnorm = 0;  // distinct sigmas
+  std::vector<SmoothPart> parts;
   GeoSmooth P{};
   GeoGrad G{};
 };
@@ -754,41 +754,51 @@ int geo_smooth_setup(satt_ctx *ctx, const char *who, const double *lons, const d
   for (int j = 0; j < ny; ++j) hd[nx + ny + j] = cosd_host(lats[j]);
   std::memcpy(hd.data() + 2 * (size_t)nx + 2 * ny, sigma, nfield * 8);
   std::vector<int> hi((size_t)nfield * (4 + ny));
-  int hx_max = 0, hy_max = 0;
+  std::vector<SmoothForm> form(nfield);
+  const double rad = 3.14159265358979323846 / 180.0;
   for (int f = 0; f < nfield; ++f) {
     // nx = sigma3/dx, ny = sigma3/cosd(lat)/dy, truncated; windows wider
     // than the grid are the same as the grid
     const double sx = sigma[f] * 3 / dx;
     hi[f] = sx < nx ? (int)sx : nx;
+    int hy_max = 0;
     for (int j = 0; j < ny; ++j) {
       const double sy = sigma[f] * 3 / cosd_host(lats[j]) / dy;
       hi[nfield + (size_t)f * ny + j] = sy >= 0 && sy < ny ? (int)sy : ny;
       hy_max = std::max(hy_max, hi[nfield + (size_t)f * ny + j]);
     }
-    hx_max = std::max(hx_max, hi[f]);
+    // the windows' largest haversine: the widest row distance and the widest
+    // column offset (at cos(lat) 1)
+    const int hx = std::min(hi[f], nx - 1);
+    double dlat = 0;
+    for (int j = 0; j < ny; ++j)
+      dlat = std::max(dlat, lats[std::min(ny - 1, j + hy_max)] - lats[j]);
+    const double sa = std::sin(std::min(dlat, 180.0) * rad / 2),
+                 so = std::sin(std::min(hx * dx, 180.0) * rad / 2);
+    form[f] = smooth_form(hx, 1.01 * (sa * sa + so * so));
   }
-  hx_max = std::min(hx_max, nx - 1);
   int *order = hi.data() + (size_t)nfield * (1 + ny);
   for (int f = 0; f < nfield; ++f) order[f] = f;
-  std::stable_sort(order, order + nfield, [&](int a, int b) { return hi[a] > hi[b]; });
+  std::stable_sort(order, order + nfield, [&](int a, int b) {
+    if (form[a].split != form[b].split) return form[a].split < form[b].split;
+    if (form[a].series != form[b].series) return !form[a].series;
+    return hi[a] > hi[b];
+  });
   // the distinct sigmas, whose weights' sums their fields share
   int *norm_of = order + nfield, *norm_field = norm_of + nfield;
   std::map<double, int> seen;
+  B.parts.clear();
   for (int q = 0; q < nfield; ++q) {
     const int f = order[q];
+    if (q == 0 || !(form[f] == form[order[q - 1]]))
+      B.parts.push_back({form[f], 0, 0, std::min(hi[f], nx - 1)});
     const auto it = seen.emplace(sigma[f], (int)seen.size());
     if (it.second) norm_field[it.first->second] = f;
     norm_of[f] = it.first->second;
+    ++B.parts.back().fields;
+    B.parts.back().norms += it.second;
   }
-  B.nnorm = (int)seen.size();
-  // a window's largest haversine: the widest row distance and the widest
-  // column offset (at cos(lat) 1)
-  double dlat = 0;
-  for (int j = 0; j < ny; ++j)
-    dlat = std::max(dlat, lats[std::min(ny - 1, j + hy_max)] - lats[j]);
-  const double rad = 3.14159265358979323846 / 180.0;
-  const double sa = std::sin(std::min(dlat, 180.0) * rad / 2),
-               so = std::sin(std::min(hx_max * dx, 180.0) * rad / 2);
+  const size_t nnorm = seen.size();
   TRY(upload(ctx, B.axes, hd.data(), hd.size() * 8));
   ALLOC(ctx, B.tab, (size_t)nx * 8 + hi.size() * sizeof(int));
   double *ax = B.axes.as<double>();
@@ -796,7 +806,7 @@ int geo_smooth_setup(satt_ctx *ctx, const char *who, const double *lons, const d
   int *dh = reinterpret_cast<int *>(s2 + nx);
   HIPCHK(ctx, hipMemcpyAsync(dh, hi.data(), hi.size() * sizeof(int), hipMemcpyHostToDevice,
                              ctx->stream));
-  ALLOC(ctx, B.out, (size_t)(nfield + B.nnorm) * N * 8);
+  ALLOC(ctx, B.out, (nfield + nnorm) * N * 8);
   launch_geo_s2(ctx->stream, ax, nx, s2);
   B.P.nx = nx;
   B.P.ny = ny;
@@ -809,8 +819,6 @@ int geo_smooth_setup(satt_ctx *ctx, const char *who, const double *lons, const d
   B.P.norm_of = B.P.order + nfield;
   B.P.norm_field = B.P.norm_of + nfield;
   B.P.den = B.out.as<double>() + (size_t)nfield * N;
-  B.P.hx_max = hx_max;
-  B.P.a_max = 1.01 * (sa * sa + so * so);
   B.P.out = B.out.as<double>();
   B.G.nx = nx;
   B.G.ny = ny;
@@ -878,7 +886,7 @@ extern "C" int satt_smooth_geo2(satt_ctx *ctx, const double *lons, const double 
   B.P.data = nat;
   GeoTimer t;
   TRY(geo_timer_start(ctx, t));
-  launch_smooth_geo2(ctx->stream, B.P, nfield, B.nnorm);
+  launch_smooth_geo2(ctx->stream, B.P, B.parts.data(), (int)B.parts.size());
   TRY(geo_timer_stop(ctx, t));
   double *res = B.out.as<double>();
   if (nfield > 1) {  // back to period-major in the input buffer's place
@@ -946,7 +954,7 @@ extern "C" int satt_topo_metric(satt_ctx *ctx, const double *lons, const double 
   B.P.data = dz.as<double>();
   GeoTimer t;
   TRY(geo_timer_start(ctx, t));
-  launch_smooth_geo2(ctx->stream, B.P, nperiod, B.nnorm);
+  launch_smooth_geo2(ctx->stream, B.P, B.parts.data(), (int)B.parts.size());
   launch_topo_metric(ctx->stream, B.G, nperiod, B.out.as<double>(), o11, o12, o22, oag);
   TRY(geo_timer_stop(ctx, t));
   HIPCHK(ctx, hipMemcpyAsync(m11, o11, M * 8, hipMemcpyDeviceToHost, ctx->stream));
@@ -982,7 +990,7 @@ extern "C" int satt_steepest_descent(satt_ctx *ctx, const double *lons, const do
   GeoTimer t;
   TRY(geo_timer_start(ctx, t));
   launch_pm_to_nat(ctx->stream, N, nperiod, din.as<double>(), nat);
-  launch_smooth_geo2(ctx->stream, B.P, nperiod, B.nnorm);
+  launch_smooth_geo2(ctx->stream, B.P, B.parts.data(), (int)B.parts.size());
   launch_to_period_major(ctx->stream, (int)N, nperiod, B.out.as<double>(), kpm);
   launch_sd_update(ctx->stream, M, kpm, updatemax, dsv.as<double>(), part);
   TRY(geo_timer_stop(ctx, t));

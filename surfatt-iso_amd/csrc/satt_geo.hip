@@ -281,6 +281,7 @@ __global__ __launch_bounds__(64 * kMaxSplit) void k_smooth_norm(GeoSmooth P, int
 // call's windows are 200 times the narrowest one's work: a wave doing one
 // alone ran 5 ms.
 // C is odd: lanes C doubles apart then read 32 different LDS bank pairs.
+constexpr size_t kLdsHalf = 80 * 1024;  // of a CU's LDS: two workgroups a CU
 constexpr int kPadC = 2;  // columns staged past the window on either side, in units of C
 // LDS doubles of one wave: the weights, the staged row
 size_t smooth_lds_doubles(int G, int C, int hxe) {
@@ -513,51 +514,53 @@ void launch_geo_s2(hipStream_t s, const double *lon, int nx, double *s2) {
   hipLaunchKernelGGL(k_geo_s2, flat_grid((size_t)nx), dim3(256), 0, s, lon, nx, s2);
 }
 
+// The waves of a workgroup: as many as leave two workgroups a CU the LDS of
+// the tile that takes the most columns (one group, C = 13).
+SmoothForm smooth_form(int hx, double a) {
+  int S = kMaxSplit;
+  while (S > 1 && S * smooth_lds_doubles(1, 13, hx) * sizeof(double) > kLdsHalf) S >>= 1;
+  return {S, a <= kSmallA};
+}
+
 namespace {
 
 template <int RN>
-void norm_launch(hipStream_t s, const GeoSmooth &P, int nnorm, int S) {
-  const size_t wave = (size_t)RN * ((P.hx_max + 1) | 1);
+void norm_launch(hipStream_t s, const GeoSmooth &P, const SmoothPart &part) {
+  const int S = part.form.split;
+  const size_t wave = (size_t)RN * ((part.hx_max + 1) | 1);
   const size_t lds = S * std::max(wave, (size_t)64 * kNormC) * sizeof(double);
-  const dim3 grid((unsigned)((P.ny + RN - 1) / RN), (unsigned)nnorm,
+  const dim3 grid((unsigned)((P.ny + RN - 1) / RN), (unsigned)part.norms,
                   (unsigned)((P.nx + 64 * kNormC - 1) / (64 * kNormC)));
-  if (P.a_max <= kSmallA)
+  if (part.form.series)
     hipLaunchKernelGGL((k_smooth_norm<RN, true>), grid, dim3(64 * S), lds, s, P, (int)wave);
   else
     hipLaunchKernelGGL((k_smooth_norm<RN, false>), grid, dim3(64 * S), lds, s, P, (int)wave);
 }
 
 template <int G, int C>
-void smooth_launch(hipStream_t s, const GeoSmooth &P, int nfield, int nnorm) {
-  // the waves of a workgroup: as many as leave two workgroups a CU
-  const size_t wave = smooth_lds_doubles(G, C, P.hx_max);
-  int S = kMaxSplit;
-  while (S > 1 && S * wave * sizeof(double) > 80 * 1024) S >>= 1;
-  if (8 * S * (P.hx_max + 2) * sizeof(double) <= 80 * 1024)
-    norm_launch<8>(s, P, nnorm, S);
-  else
-    norm_launch<1>(s, P, nnorm, S);
+void tile_launch(hipStream_t s, const GeoSmooth &P, const SmoothPart &part) {
+  const int S = part.form.split;
+  const size_t wave = smooth_lds_doubles(G, C, part.hx_max);
   const size_t sums = (size_t)(S - 1) * 2 * C * 64;
   const size_t lds = std::max(S * wave, sums) * sizeof(double);
   constexpr int kTile = 64 / G * C;
-  const dim3 grid((unsigned)((P.ny + 2 * G - 1) / (2 * G)), (unsigned)nfield,
+  const dim3 grid((unsigned)((P.ny + 2 * G - 1) / (2 * G)), (unsigned)part.fields,
                   (unsigned)((P.nx + kTile - 1) / kTile));
-  if (P.a_max <= kSmallA)
+  if (part.form.series)
     hipLaunchKernelGGL((k_smooth_geo2<G, C, true>), grid, dim3(64 * S), lds, s, P, (int)wave);
   else
     hipLaunchKernelGGL((k_smooth_geo2<G, C, false>), grid, dim3(64 * S), lds, s, P, (int)wave);
 }
 
-}  // namespace
-
 // The tile (G lane groups, C columns a lane) whose columns cover a row with
-// the fewest idle lanes; at equal cover the wider C.  Windows whose weights
-// of 2G rows and staged row pass 64 KB take one group.
-void launch_smooth_geo2(hipStream_t s, const GeoSmooth &P, int nfield, int nnorm) {
+// the fewest idle lanes; at equal cover the wider C.  More than one group
+// where the weights of 2G rows and the staged row leave two workgroups a CU.
+void part_launch(hipStream_t s, const GeoSmooth &P, const SmoothPart &part) {
+  const int S = part.form.split;
   int bg = 1, bc = 13, cover = INT_MAX;
   for (int C : {13, 11, 9})
     for (int G : {1, 2, 4}) {
-      if (G > 1 && smooth_lds_doubles(G, C, P.hx_max) * sizeof(double) > 64 * 1024) continue;
+      if (G > 1 && S * smooth_lds_doubles(G, C, part.hx_max) * sizeof(double) > kLdsHalf) continue;
       const int tile = 64 / G * C, n = (P.nx + tile - 1) / tile * tile;
       if (n < cover) {
         cover = n;
@@ -568,11 +571,11 @@ void launch_smooth_geo2(hipStream_t s, const GeoSmooth &P, int nfield, int nnorm
   auto go = [&](auto c) {
     constexpr int C = decltype(c)::value;
     if (bg == 1)
-      smooth_launch<1, C>(s, P, nfield, nnorm);
+      tile_launch<1, C>(s, P, part);
     else if (bg == 2)
-      smooth_launch<2, C>(s, P, nfield, nnorm);
+      tile_launch<2, C>(s, P, part);
     else
-      smooth_launch<4, C>(s, P, nfield, nnorm);
+      tile_launch<4, C>(s, P, part);
   };
   if (bc == 13)
     go(std::integral_constant<int, 13>{});
@@ -580,6 +583,25 @@ void launch_smooth_geo2(hipStream_t s, const GeoSmooth &P, int nfield, int nnorm
     go(std::integral_constant<int, 11>{});
   else
     go(std::integral_constant<int, 9>{});
+}
+
+}  // namespace
+
+void launch_smooth_geo2(hipStream_t s, GeoSmooth P, const SmoothPart *parts, int nparts) {
+  double *den = P.den;
+  for (int q = 0; q < nparts; ++q) {
+    const SmoothPart &part = parts[q];
+    GeoSmooth N = P;  // the sums of the part's own sigmas
+    N.den = den;
+    if ((size_t)part.form.split * 8 * (part.hx_max + 2) * sizeof(double) <= kLdsHalf)
+      norm_launch<8>(s, N, part);
+    else
+      norm_launch<1>(s, N, part);
+    part_launch(s, P, part);
+    den += (size_t)part.norms * P.nx * P.ny;
+    P.order += part.fields;
+    P.norm_field += part.norms;
+  }
 }
 
 void launch_gradient_geo2(hipStream_t s, const GeoGrad &G, int nf, const double *f_nat,

@@ -199,13 +199,28 @@ struct GeoSmooth {
   const double *s2;             // sin((lon(k)-lon(0))*deg2rad/2)**2, k < nx
   const double *data, *sigma;
   const int *hx, *hy;
-  const int *order;             // the fields, widest window first
+  const int *order;             // the fields, part after part, widest window first
   const int *norm_of;           // each field's distinct sigma
-  const int *norm_field;        // a field of each distinct sigma, widest first
+  const int *norm_field;        // a field of each distinct sigma, in the order of the fields
   double *den;                  // [distinct sigma][j][i]: the weights' sums
-  int hx_max;                   // widest half-width, at most nx - 1
-  double a_max;                 // bound on sin(theta/2)**2 over every window
   double *out;                  // [f][j][i]
+};
+// What the rounding of a field's sums depends on, by its own windows alone, so
+// that a field smoothed alone and beside others is the same: the waves that
+// split its window rows, and whether its weights take the power series.
+struct SmoothForm {
+  int split;
+  bool series;
+  bool operator==(const SmoothForm &o) const { return split == o.split && series == o.series; }
+};
+// hx: half-width, at most nx - 1; a: bound on sin(theta/2)**2 over the windows
+SmoothForm smooth_form(int hx, double a);
+// Fields of one form, one after another in GeoSmooth::order: a launch of each
+// kernel.
+struct SmoothPart {
+  SmoothForm form;
+  int fields, norms;            // how many, and of how many sigmas
+  int hx_max;                   // their widest half-width, at most nx - 1
 };
 struct GeoGrad {
   int nx, ny;
@@ -213,7 +228,7 @@ struct GeoGrad {
   const double *cosd_lat;       // cosd(lat(j)), host-computed
 };
 void launch_geo_s2(hipStream_t s, const double *lon, int nx, double *s2);
-void launch_smooth_geo2(hipStream_t s, const GeoSmooth &P, int nfield, int nnorm);
+void launch_smooth_geo2(hipStream_t s, GeoSmooth P, const SmoothPart *parts, int nparts);
 // tx, ty period-major (nf, nx, ny) of nf natural fields
 void launch_gradient_geo2(hipStream_t s, const GeoGrad &G, int nf, const double *f_nat,
                           double *tx_pm, double *ty_pm);

@@ -94,6 +94,21 @@ def test_smoothing_tiles_match_oracle(ctx, nx, ny, d, sigmas):
     assert np.all(ones == 1.0)
 
 
+@pytest.mark.parametrize("nx,ny,d,sigmas", [
+    (1100, 5, 0.002, [0.02, 0.3, 0.02, 0.8]),   # rows split over four, two and one waves
+    (450, 5, 0.05, [0.5, 4.0]),                 # with and without the series of asin^2
+    (60, 41, 1.0, [8.0, 0.4, 2.0]),
+])
+def test_a_smoothed_field_does_not_depend_on_its_neighbours(ctx, nx, ny, d, sigmas):
+    lons, lats = axes(nx, ny, d)
+    data = field(nx, ny, nx, len(sigmas))
+    both = ctx.smooth_geo2(lons, lats, data, sigmas)
+    for f, s in enumerate(sigmas):
+        alone = ctx.smooth_geo2(lons, lats, data[f], s)
+        np.testing.assert_array_equal(both[f], alone)
+        smooth_close(alone, O.smooth_geo2(lons, lats, data[f], s), data[f])
+
+
 def test_smoothing_keeps_nan_and_infinity_in_their_windows(ctx):
     lons, lats = axes(150, 37, 0.02)
     z = field(150, 37, 11)
