@@ -282,6 +282,7 @@ __global__ __launch_bounds__(64 * kMaxSplit) void k_smooth_norm(GeoSmooth P, int
 // alone ran 5 ms.
 // C is odd: lanes C doubles apart then read 32 different LDS bank pairs.
 constexpr size_t kLdsHalf = 80 * 1024;  // of a CU's LDS: two workgroups a CU
+constexpr size_t kCus = 256;
 constexpr int kPadC = 2;  // columns staged past the window on either side, in units of C
 // LDS doubles of one wave: the weights, the staged row
 size_t smooth_lds_doubles(int G, int C, int hxe) {
@@ -552,22 +553,43 @@ void tile_launch(hipStream_t s, const GeoSmooth &P, const SmoothPart &part) {
     hipLaunchKernelGGL((k_smooth_geo2<G, C, false>), grid, dim3(64 * S), lds, s, P, (int)wave);
 }
 
-// The tile (G lane groups, C columns a lane) whose columns cover a row with
-// the fewest idle lanes; at equal cover the wider C.  More than one group
-// where the weights of 2G rows and the staged row leave two workgroups a CU.
+int ceil_div(int a, int b) { return (a + b - 1) / b; }
+
+// The tile of G lane groups and C columns a lane.  Where one workgroup a CU
+// does, the narrowest C, in one group or two: the call is then as long as a
+// workgroup, and its weights are of 2G rows.  Else the one whose columns cover
+// a row with the fewest idle lanes, at equal cover the wider C and fewer groups.
+// More than one group where the weights of 2G rows and the staged row leave
+// two workgroups a CU.
+// MI355X, numerators in us, windows of 25 / 121 columns, (2,13) is G = 2, C = 13:
+//   401^2, 1 field    (1,9)  40 / 235   (2,9)  41 / 238   (2,13)  56 / 314   (4,9)  48 / 265
+//   401^2, 20 fields  (1,9) 282 / 2916  (2,9) 304 / 2985  (2,13) 221 / 2186  (4,9) 305 / 2531
+//   300^2, 20 fields  (1,9) 196 / 1927  (2,11) 136 / 1227 (2,13) 160 / 1456  (4,9) 218 / 1635
+//   200^2, 1 field    (1,9)  33 / 213   (2,9)  37 / 222   (4,9)   46 / 255   (4,13) 59 / 333
+//   200^2, 20 fields  (1,9) 129 / 1143  (2,9)  84 / 714   (4,9)  105 / 742   (4,13) 76 / 541
+//   100^2, 20 fields  (1,9)  66 / 504   (2,9)  43 / 288   (4,9)   50 / 248   (4,13) 64 / 333
 void part_launch(hipStream_t s, const GeoSmooth &P, const SmoothPart &part) {
   const int S = part.form.split;
-  int bg = 1, bc = 13, cover = INT_MAX;
-  for (int C : {13, 11, 9})
-    for (int G : {1, 2, 4}) {
-      if (G > 1 && S * smooth_lds_doubles(G, C, part.hx_max) * sizeof(double) > kLdsHalf) continue;
-      const int tile = 64 / G * C, n = (P.nx + tile - 1) / tile * tile;
-      if (n < cover) {
-        cover = n;
-        bg = G;
-        bc = C;
+  auto fits = [&](int G, int C) {
+    return G == 1 || S * smooth_lds_doubles(G, C, part.hx_max) * sizeof(double) <= kLdsHalf;
+  };
+  int bg = 0, bc = 9;
+  for (int G : {1, 2})
+    if (bg == 0 && fits(G, 9) &&
+        (size_t)ceil_div(P.ny, 2 * G) * part.fields * ceil_div(P.nx, 64 / G * 9) <= kCus)
+      bg = G;
+  if (bg == 0) {
+    int cover = INT_MAX;
+    for (int C : {13, 11, 9})
+      for (int G : {1, 2, 4}) {
+        const int tile = 64 / G * C, n = ceil_div(P.nx, tile) * tile;
+        if (fits(G, C) && n < cover) {
+          cover = n;
+          bg = G;
+          bc = C;
+        }
       }
-    }
+  }
   auto go = [&](auto c) {
     constexpr int C = decltype(c)::value;
     if (bg == 1)
@@ -593,10 +615,18 @@ void launch_smooth_geo2(hipStream_t s, GeoSmooth P, const SmoothPart *parts, int
     const SmoothPart &part = parts[q];
     GeoSmooth N = P;  // the sums of the part's own sigmas
     N.den = den;
-    if ((size_t)part.form.split * 8 * (part.hx_max + 2) * sizeof(double) <= kLdsHalf)
-      norm_launch<8>(s, N, part);
-    else
+    // Rows a workgroup: few where one a CU does, else four, two where the
+    // weights of four leave less than two workgroups a CU.  MI355X, windows of
+    // 121 columns, 4 / 2 / 1 rows: one sigma on 200^2 95 / 69 / 56 us, on 401^2
+    // 98 / 70 / 89, 20 sigmas on 401^2 518 / 686 / 1135 (8 rows: 199, 202, 856).
+    const size_t rows = (size_t)P.ny * part.norms * ceil_div(P.nx, 64 * kNormC);
+    if (rows <= kCus)
       norm_launch<1>(s, N, part);
+    else if (rows <= 2 * kCus ||
+             (size_t)part.form.split * 4 * (part.hx_max + 2) * sizeof(double) > kLdsHalf)
+      norm_launch<2>(s, N, part);
+    else
+      norm_launch<4>(s, N, part);
     part_launch(s, P, part);
     den += (size_t)part.norms * P.nx * P.ny;
     P.order += part.fields;

@@ -74,11 +74,13 @@ def test_smoothing_is_deterministic_and_keeps_constants(ctx):
 
 @pytest.mark.parametrize("nx,ny,d,sigmas", [
     (2, 2, 0.05, [0.02, 0.3]),            # the smallest grid
-    (144, 5, 0.02, [0.03, 0.1, 0.03]),    # four lane groups, a full tile; two fields of one sigma
-    (145, 9, 0.02, [0.05]),               # one column past it
-    (416, 6, 0.005, [0.05, 0.2]),         # two groups, a full tile, rows a multiple of neither
+    (144, 5, 0.02, [0.03, 0.1, 0.03]),    # few workgroups: one lane group; two fields of one sigma
+    (577, 5, 0.02, [0.05]),               # one column past its tile
+    (145, 9, 0.02, [0.05]),
+    (416, 6, 0.005, [0.05, 0.2]),
     (417, 3, 0.005, [0.02]),
-    (833, 3, 0.002, [0.3]),               # one group, two tiles, windows wider than the grid
+    (20, 301, 0.02, [0.06]),              # denominators of two rows a workgroup
+    (833, 3, 0.002, [0.3]),               # windows wider than the grid
     (2600, 2, 0.001, [2.0]),              # the weights leave one wave a workgroup
     (40, 12, 1.5, [6.0, 9.0]),            # distances past the series of asin^2
 ])
@@ -92,6 +94,19 @@ def test_smoothing_tiles_match_oracle(ctx, nx, ny, d, sigmas):
         smooth_close(out[f], O.smooth_geo2(lons, lats, data[f], s), data[f])
     ones = ctx.smooth_geo2(lons, lats, np.ones((nx, ny)), sigmas)
     assert np.all(ones == 1.0)
+
+
+@pytest.mark.parametrize("nx", [41, 144, 145, 208, 288, 289, 353, 416, 417, 600])
+def test_smoothing_of_many_fields_matches_oracle(ctx, nx):
+    """Workgroups enough to fill the chip: the tiles of two and four lane groups,
+    full and with one column past them, and rows that leave a remainder."""
+    ny, nf = 59, 18
+    lons, lats = axes(nx, ny, 0.02)
+    data, sigmas = field(nx, ny, nx, nf), 0.03 + 0.005 * np.arange(nf)
+    out = ctx.smooth_geo2(lons, lats, data, sigmas)
+    for f in (0, 7, nf - 1):
+        smooth_close(out[f], O.smooth_geo2(lons, lats, data[f], sigmas[f]), data[f])
+    assert np.all(ctx.smooth_geo2(lons, lats, np.ones((nx, ny)), sigmas) == 1.0)
 
 
 @pytest.mark.parametrize("nx,ny,d,sigmas", [
