@@ -160,8 +160,12 @@ struct LatTerms {
   }
 };
 
+// kap, finite where 2 sigma^2 is not 0 (it overflows below sigma = 6e-153): the
+// weight of the cell itself is then 1, as the quotient of its distance gives it.
 __device__ __forceinline__ double geo_kap(double sig) {
-  return 4.0 * (kGeoRadius * kGeoKm2Deg) * (kGeoRadius * kGeoKm2Deg) / (2.0 * (sig * sig));
+  const double two = 2.0 * (sig * sig);
+  const double kap = 4.0 * (kGeoRadius * kGeoKm2Deg) * (kGeoRadius * kGeoKm2Deg) / two;
+  return two > 0.0 ? fmin(kap, 1.7976931348623157e308) : kap;
 }
 // the wave sw's first window row at or after n1
 __device__ __forceinline__ int first_row(int n1, int sw, int S) {

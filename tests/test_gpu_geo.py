@@ -124,6 +124,15 @@ def test_a_smoothed_field_does_not_depend_on_its_neighbours(ctx, nx, ny, d, sigm
         smooth_close(alone, O.smooth_geo2(lons, lats, data[f], s), data[f])
 
 
+@pytest.mark.parametrize("sigma", [1e-150, 1e-154, 1e-160])
+def test_smoothing_with_the_smallest_sigmas_keeps_the_field(ctx, sigma):
+    """Windows of one cell, whose weight is 1 while sigma^2 is not 0."""
+    lons, lats = axes(20, 11, 0.05)
+    data = field(20, 11, 3)
+    np.testing.assert_array_equal(O.smooth_geo2(lons, lats, data, sigma), data)
+    np.testing.assert_array_equal(ctx.smooth_geo2(lons, lats, data, sigma), data)
+
+
 def test_smoothing_keeps_nan_and_infinity_in_their_windows(ctx):
     lons, lats = axes(150, 37, 0.02)
     z = field(150, 37, 11)
