@@ -9,6 +9,7 @@ difference quotients over +-0.5% in period, which amplify that about 100-fold.""
 import numpy as np
 import pytest
 
+import oracle as O
 import satt
 
 pytestmark = pytest.mark.gpu
@@ -40,8 +41,8 @@ def test_roots_do_not_depend_on_the_steps_before_them(ctx, iwave, igr, nz, top):
 
 
 def test_columns_without_a_root_are_still_reported(ctx):
-    """A soft layer under a stiff lid: the fundamental mode leaves the search's
-    range, with the columns beside it unaffected."""
+    """A column of NaN, whose period equation never changes sign, with the
+    columns beside it unaffected."""
     vs, z = columns(3, 2, 20, 3.0, 5)
     good = ctx.fwdsurf3d(vs, z, [5.0, 20.0])
     bad = vs.copy(order="F")
@@ -53,3 +54,42 @@ def test_columns_without_a_root_are_still_reported(ctx):
     keep = np.ones((3, 2), bool)
     keep[1, 1] = False
     assert np.array_equal(out[:, keep], good[:, keep])
+
+
+def test_search_that_leaves_its_range_is_reported(ctx):
+    """A homogeneous half-space carries no Love wave: at a wavelength of seven
+    times the model's depth (past what the flattened earth's curvature traps)
+    no step up to the largest Vs changes the sign.  The last step of the range
+    lies among the first 64 (0.87 to 1.01 of Vs 1.5), or several rounds up."""
+    for vs in (1.5, 4.0):
+        out, good = {}, columns(3, 2, 20, 3.0, 5)[0]
+        _, z = columns(1, 1, 20, 3.0, 5)
+        mixed = good.copy(order="F")
+        mixed[2, 0, :] = vs
+        for p in ([5.0], [420.0 / vs]):
+            ref = ctx.fwdsurf3d(good, z, p, 1, 0)
+            out, st = ctx.fwdsurf3d(mixed, z, p, 1, 0, status=True)
+            if p[0] > 5.0:
+                assert st[2, 0] == satt.E_DISPERSION and out[0, 2, 0] == 0
+            else:
+                assert st[2, 0] == 0
+            st[2, 0] = 0
+            assert not st.any()
+            keep = np.ones((3, 2), bool)
+            keep[2, 0] = False
+            assert np.array_equal(out[:, keep], ref[:, keep])
+
+
+@pytest.mark.parametrize("vs", [1.5, 2.0, 4.0])
+def test_root_and_limit_among_the_same_steps(ctx, vs):
+    """The Rayleigh velocity of a homogeneous half-space, from its own equation
+    (a tolerance of 1e-3 for the flattening of the earth, a wavelength over its
+    radius): the search starts at 0.95 of it, and for the lower velocities the
+    limit above Vs is among the 64 steps that bracket it, after it."""
+    vp = float(O.brocher_vp_rho(np.float32(vs))[0])
+    c = np.linspace(0.7, 0.9999, 200001) * vs
+    f = (2 - (c / vs) ** 2) ** 2 - 4 * np.sqrt(1 - (c / vp) ** 2) * np.sqrt(1 - (c / vs) ** 2)
+    root = c[np.argmax(np.sign(f) != np.sign(f[0]))]
+    z = np.linspace(0.0, 60.0, 20)
+    got = ctx.fwdsurf3d(np.full((2, 2, 20), vs, order="F"), z, [1.0, 2.0])
+    assert np.all(np.abs(got - root) < 1e-3 * root)
