@@ -309,6 +309,11 @@ int satt_hbm_probe(satt_ctx *ctx, double nbytes, double *read_gbs, double *copy_
  * 256 bytes per clock per CU (gfx950) at the device's clock, both in GB/s.  A
  * measurement aid; no counterpart in the reference. */
 int satt_lds_probe(satt_ctx *ctx, double *read_gbs, double *peak_gbs);
+/* The sweeps' own quotients and roots of n operands, for tests: out = x / y
+ * (op 0), 1 / x (1) or sqrt(x) (2), in FP64, or with single != 0 in FP32 on
+ * operands rounded to it. */
+int satt_div_probe(satt_ctx *ctx, int op, int single, int n, const double *x,
+                   const double *y, double *out);
 
 /* Device time in ms of the kernels of the last satt_smooth_geo2,
  * satt_gradient_geo2, satt_topo_metric, satt_steepest_descent,

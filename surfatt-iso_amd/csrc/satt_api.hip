@@ -856,6 +856,23 @@ extern "C" int satt_lds_probe(satt_ctx *ctx, double *read_gbs, double *peak_gbs)
   return SATT_OK;
 }
 
+extern "C" int satt_div_probe(satt_ctx *ctx, int op, int single, int n, const double *x,
+                              const double *y, double *out) {
+  if (!ctx) return SATT_E_ARG;
+  if (op < 0 || op > 2 || n < 1 || !x || !y || !out)
+    return fail(ctx, SATT_E_ARG, "satt_div_probe: bad arguments");
+  HIPCHK(ctx, hipSetDevice(ctx->device));
+  const size_t N = (size_t)n;
+  DBuf dx, dy, res;
+  TRY(upload(ctx, dx, x, N * 8));
+  TRY(upload(ctx, dy, y, N * 8));
+  ALLOC(ctx, res, N * 8);
+  launch_div_probe(ctx->stream, op, single != 0, N, dx.as<double>(), dy.as<double>(),
+                   res.as<double>());
+  HIPCHK(ctx, hipMemcpyAsync(out, res.p, N * 8, hipMemcpyDeviceToHost, ctx->stream));
+  return sync_status(ctx);
+}
+
 extern "C" double satt_topo_sigma(double vel, double period, double wavelen_factor) {
   const double pi = (double)3.14159265359f;
   const double km2deg = 1.0 / (6371.0 * pi / 180.0);

@@ -292,6 +292,10 @@ struct DispJob {
 int stream_probe(hipStream_t s, int cus, size_t nbytes, int reps, double &read_gbs,
                  double &copy_gbs);
 int lds_probe(hipStream_t s, int cus, int reps, double &read_gbs);
+// out[k] = x[k] / y[k] (op 0), 1 / x[k] (1) or sqrt(x[k]) (2), as satt_div.h
+// forms them, in float if `single`
+void launch_div_probe(hipStream_t s, int op, bool single, size_t n, const double *x,
+                      const double *y, double *out);
 // LDS of one column's wave (the layered model and the per-layer terms) for
 // n layers
 size_t fwdsurf_lds_bytes(int n);

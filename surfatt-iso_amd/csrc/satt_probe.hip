@@ -3,10 +3,12 @@
 // a read-only sum and a copy; and achievable LDS read bandwidth (16-byte LDS
 // reads of every thread of four workgroups per CU).  Measurement aids for the
 // roofline of the path's kernels; they have no counterpart in the reference.
+// And the sweeps' quotients and roots (satt_div.h) of given operands, for tests.
 #include <hip/hip_runtime.h>
 
 #include <vector>
 
+#include "satt_div.h"
 #include "satt_internal.h"
 
 namespace satt {
@@ -54,7 +56,24 @@ __global__ void k_stream_fill(float4 *p, size_t n) {
     p[i] = make_float4(1.0f, 2.0f, 3.0f, 4.0f);
 }
 
+template <typename V>
+__device__ __forceinline__ V div_op(int op, V x, V y) {
+  return op == 0 ? quot(x, recip_of(y)) : op == 1 ? inverse(x) : root_of(x);
+}
+__global__ __launch_bounds__(256) void k_div_probe(int op, int single, size_t n, const double *x,
+                                                   const double *y, double *out) {
+  const size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  out[k] = single ? (double)div_op(op, (float)x[k], (float)y[k]) : div_op(op, x[k], y[k]);
+}
+
 }  // namespace
+
+void launch_div_probe(hipStream_t s, int op, bool single, size_t n, const double *x,
+                      const double *y, double *out) {
+  hipLaunchKernelGGL(k_div_probe, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, op,
+                     (int)single, n, x, y, out);
+}
 
 int stream_probe(hipStream_t s, int cus, size_t nbytes, int reps, double &read_gbs,
                  double &copy_gbs) {

@@ -426,6 +426,15 @@ class Context:
         self._check(self.lib.satt_lds_probe(self.ptr, ctypes.byref(r), ctypes.byref(pk)))
         return r.value, pk.value
 
+    def div_probe(self, op, x, y=None, single=False):
+        """x / y (op 0), 1 / x (1) or sqrt(x) (2) as the sweeps form them."""
+        x = _c(x)
+        y = x if y is None else _c(y)
+        out = np.empty_like(x)
+        self._check(self.lib.satt_div_probe(self.ptr, int(op), int(single), x.size, _d(x), _d(y),
+                                            _d(out)))
+        return out
+
     def last_device_ms(self):
         """Device time of the last model-side call's kernels (ms)."""
         return float(self.lib.satt_last_device_ms(self.ptr))
