@@ -48,6 +48,11 @@
  *     returns them silently (src/eikon_solver_2d.f90:1117-1119,1436-1438).
  *   - A context owns one HIP stream on one device and is not thread-safe;
  *     use one context per host thread.
+ *   - Quotients and square roots in the sweeps are correctly rounded while
+ *     operands and results are within 2^-500 .. 2^500 (FP64) and 2^-90 .. 2^90
+ *     (the mixed mode's FP32).  They are of the size of (time / spacing in
+ *     radians)^4 and ^2 or less: 2^104 and 2^52 for 1000 s at 0.001 degrees.
+ *     Zeros, infinities and NaN are IEEE's.
  */
 #ifndef SATT_H
 #define SATT_H
@@ -107,7 +112,13 @@ const char *satt_version(void);
 
 /* ---------------------------------------------------- per-solve (plain) form
  * One solve per launch; host arrays in and out.  `iters` (may be NULL)
- * receives the iteration count at exit. */
+ * receives the iteration count at exit.
+ * satt_fwd_lonlat and satt_adj_lonlat choose the kernels by the grid's size:
+ * one solve across compute units, the batched sweeps, or one workgroup; the
+ * fields and counts are the same bits.  A context keeps their scratch, up to
+ * 256 MB of device memory (a forward takes about 1000 bytes a cell), until
+ * satt_destroy; a larger one is given back at the end of the call.  They do
+ * not return SATT_E_TEAM_WAIT: a solve whose waits ran out is done again. */
 
 /* FSM_UW_PS_lonlat_2d(xx_deg,yy_deg,nx,ny,spha,sphb,sphc,T,fun,x0_deg,y0_deg,u)
  * src/eikon_solver_2d.f90:764.  `u` only feeds an unused error norm in the
@@ -132,8 +143,9 @@ int satt_adj_lonlat(satt_ctx *ctx, const double *xx_deg, const double *yy_deg,
  * counts as one whose waits did.  The results do not change. */
 int satt_solve_fail_waits(satt_ctx *ctx, int strip, int team);
 
-/* satt_fwd_lonlat without any device allocation: the same kernels on the same
- * operands, hence the same T bit for bit.  No counterpart in the reference;
+/* satt_fwd_lonlat without any device allocation, always on the one-workgroup
+ * kernels: the same T bit for bit, as the tests hold it, in about ten times the
+ * time on a 401 x 343 grid.  No counterpart in the reference;
  * it is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Its work
  * space is one static device array per GPU (about 28 MB, held until the

@@ -1,7 +1,7 @@
 // The allocation-free per-solve forward solve, satt_fwd_lonlat_noalloc
-// (include/satt.h): the kernels of satt_fwd_lonlat on the same operands, with
-// every device buffer beyond the caller's arrays carved from one file-scope
-// device array instead of hipMalloc.
+// (include/satt.h): the one-workgroup kernels, which give satt_fwd_lonlat's
+// fields bit for bit, with every device buffer beyond the caller's arrays carved
+// from one file-scope device array instead of hipMalloc.
 //
 // Each GPU the library runs on holds its own copy of the array for the life
 // of the process.  Host code never passes the array's name to a kernel or a
