@@ -116,9 +116,10 @@ const char *satt_version(void);
  * satt_fwd_lonlat and satt_adj_lonlat choose the kernels by the grid's size:
  * one solve across compute units, the batched sweeps, or one workgroup; the
  * fields and counts are the same bits.  A context keeps their scratch, up to
- * 256 MB of device memory (a forward takes about 1000 bytes a cell), until
- * satt_destroy; a larger one is given back at the end of the call.  They do
- * not return SATT_E_TEAM_WAIT: a solve whose waits ran out is done again. */
+ * 256 MB of device memory (a forward takes about 1000 bytes a cell, an adjoint
+ * 480), until satt_destroy; a larger one is given back at the end of the call.
+ * They do not return SATT_E_TEAM_WAIT: a solve whose waits ran out is done
+ * again. */
 
 /* FSM_UW_PS_lonlat_2d(xx_deg,yy_deg,nx,ny,spha,sphb,sphc,T,fun,x0_deg,y0_deg,u)
  * src/eikon_solver_2d.f90:764.  `u` only feeds an unused error norm in the

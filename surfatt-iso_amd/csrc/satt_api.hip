@@ -377,7 +377,7 @@ int strip_solve_setup(satt_ctx *ctx, StripSolve &S, const double *xd, const doub
   const size_t o_trig = c.take(2 * (size_t)ny * 8), o_in = c.take(4 * N * 8);
   const size_t o_abc = c.take(3 * N * 8), o_ps = c.take(2 * (size_t)kPF * SE * 8);
   const size_t o_slot = c.take(slot_doubles(nx, ny, kSlotSkews) * 8);
-  const size_t o_quad = c.take(quad ? quad_scratch_bytes(nx, ny) : 0);
+  const size_t o_quad = c.take(quad ? quad_scratch_bytes(nx, ny, !fun) : 0);
   char *ws = solve_scratch(ctx, c.at);
   if (!ws) return 1;
   std::vector<char> h(sizeof(SolveItem) + (nax + 3 * (size_t)nr) * 8);

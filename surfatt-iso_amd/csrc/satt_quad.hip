@@ -501,7 +501,7 @@ bool quad_fits(int nx, int ny) {
 namespace {
 struct QuadLayout {
   size_t rec, t0, snap, chan, conv, stop, total;
-  QuadLayout(int nx, int ny) {
+  QuadLayout(int nx, int ny, bool adj) {
     const size_t ns = (nx + kCols - 1) / kCols, n = ns * ny;
     size_t at = 0;
     auto take = [&](size_t bytes) {
@@ -509,7 +509,7 @@ struct QuadLayout {
       at = (at + bytes + 255) & ~(size_t)255;
       return o;
     };
-    rec = take(n * 64 * kRec * 8);
+    rec = take(n * (adj ? kCols * kRecA : 64 * kRec) * 8);
     t0 = take((size_t)nx * ny * 8);
     snap = take(n * kCols * 8);
     chan = take(n * 8 * 8);  // [2][ns][2][ny][2]
@@ -520,11 +520,11 @@ struct QuadLayout {
 };
 }  // namespace
 
-size_t quad_scratch_bytes(int nx, int ny) { return QuadLayout(nx, ny).total; }
+size_t quad_scratch_bytes(int nx, int ny, bool adj) { return QuadLayout(nx, ny, adj).total; }
 
 namespace {
-Quad quad_of(const SlotDesc &D, void *scratch, int quit) {
-  const QuadLayout L(D.g.nx, D.g.ny);
+Quad quad_of(const SlotDesc &D, bool adj, void *scratch, int quit) {
+  const QuadLayout L(D.g.nx, D.g.ny, adj);
   char *b = static_cast<char *>(scratch);
   Quad Q;
   Q.nx = D.g.nx;
@@ -551,7 +551,7 @@ void quad_clear(hipStream_t s, const Quad &Q) {
 
 void launch_fwd_quad(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, const SlotDesc &D,
                      const PeriodFields &pf, void *scratch, int quit) {
-  const Quad Q = quad_of(D, scratch, quit);
+  const Quad Q = quad_of(D, false, scratch, quit);
   const size_t lanes = (size_t)Q.ns * Q.ny * 64;
   launch_fwd_prep(s, sd, gd);
   quad_clear(s, Q);
@@ -563,7 +563,7 @@ void launch_fwd_quad(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, con
 
 void launch_adj_quad(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, const SlotDesc &D,
                      const PeriodFields &pf, void *scratch, int quit) {
-  const Quad Q = quad_of(D, scratch, quit);
+  const Quad Q = quad_of(D, true, scratch, quit);
   const size_t SE = D.sg.skew_elems(), cells = (size_t)Q.ns * Q.ny * kCols;
   launch_zero(s, D.skew + 5 * SE, SE * 8);
   launch_adj_source(s, sd, gd, 0, false);

@@ -154,7 +154,7 @@ __device__ __forceinline__ size_t skpos(int sk, int i, int j, int R) {
 // strip that gives up at its end (for tests), or -1.
 constexpr int kQuadMaxStrips = 64;  // waves of a launch: a quarter of the CUs
 bool quad_fits(int nx, int ny);
-size_t quad_scratch_bytes(int nx, int ny);
+size_t quad_scratch_bytes(int nx, int ny, bool adj);
 void launch_fwd_quad(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, const SlotDesc &D,
                      const PeriodFields &pf, void *scratch, int quit);
 void launch_adj_quad(hipStream_t s, const SlotDesc *sd, const GroupDims &gd, const SlotDesc &D,
