@@ -275,9 +275,9 @@ __global__ __launch_bounds__(64 * kMaxSplit) void k_smooth_norm(GeoSmooth P, int
 // the form before it (a thread per column of two rows) took a product and two
 // sums a node and 1.5 LDS reads of 8 bytes.  With C = 7 and one group the
 // reads still bound it: C = 13 and two groups halve them per node.
-// MI355X, 401^2 at 0.005 degrees: smoothing of 20 kernels at sigma 0.2 8.3 ms
-// and 0.5 for the denominators, against 33.6, the metric's 20 periods 6.2 and
-// 1.5 ms against 29.9; at the 65 TFLOP/s that independent FP64 multiply-adds
+// MI355X, 401^2 at 0.005 degrees: smoothing of 20 kernels at sigma 0.2 8.1 ms
+// and 0.2 for the denominators, against 33.6, the metric's 20 periods 6.3 and
+// 1.1 ms against 29.9; at the 65 TFLOP/s that independent FP64 multiply-adds
 // reach they are 4.4 and 3.2 ms.  What is left is issue: the vector units are
 // busy two thirds of the cycles, a quarter of that with the weights, the
 // zeroing and adding of the sums and the staging of each row, at a clock
